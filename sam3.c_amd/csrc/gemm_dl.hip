@@ -934,8 +934,17 @@ extern "C" int s3k_dl_eligible(const struct s3k_gemm *g)
  *   - 192x128 (cfg 24 / 10, 8 waves) when that gives at least 192 tiles
  *     (fc2, proj, batched attention), and first of all for N <= 128 (P V
  *     as an NT product: 200 against 303 us for 192x256);
- *   - 128x128 (cfg 4, 4 waves) for mid-size problems, 64x64 (cfg 2) for
- *     small ones.
+ *   - 64x64 tiles of 64-k steps up to 768 of them (at most three per CU,
+ *     all resident): a ring of four stages (cfg 5, 64 KiB, two workgroups
+ *     per CU) up to 512, of three (cfg 14, three per CU) above. Such a
+ *     problem is bound by how many bytes a CU keeps in flight towards L2
+ *     and by CUs without a tile, not by the MFMAs: 1369x1000x1544 f16
+ *     (352 tiles) 23.0 us on 88 tiles of 128x128 with one step in flight,
+ *     13.6 here; 576x1024x4096 31.8 -> 20.2 (144 tiles), 169x768x3072
+ *     24.9 -> 15.5 (36), 5184x512x512 8.1 -> 7.0 (648). Past 768 tiles
+ *     the larger tiles' fewer L2 bytes win (2500x2048x512, 1280 tiles:
+ *     10.7 here, 9.6 on 192x128);
+ *   - 128x128 (cfg 4, 4 waves) between that and 192 tiles of 192x128.
  *   - K = 64 with M, N multiples of 192 and at least 1024 such tiles
  *     (attention scores over many slices): the persistent gemm_dlk,
  *     six waves (cfg 30; cfg 31 the four-wave form, as fast within the
@@ -956,7 +965,10 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 	if (cfg < 0) {
 		const long long t9 = dl_tiles(g, 256, 256), t10 = dl_tiles(g, 192, 128);
 		const bool pipe = g->K % 64 == 0;
-		if (pipe && g->N <= 128 && t10 >= 192)
+		const long long t5 = dl_tiles(g, 64, 64);
+		if (t5 <= 768)
+			cfg = t5 <= 512 ? 5 : 14;
+		else if (pipe && g->N <= 128 && t10 >= 192)
 			cfg = 24; /* narrow N: wider tiles would only compute padding */
 		else if (t9 >= 224 && t9 <= 256)
 			cfg = pipe ? 20 : 9;
@@ -966,10 +978,8 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 			cfg = 23;
 		else if (t10 >= 192)
 			cfg = pipe ? 24 : 10;
-		else if (dl_tiles(g, 128, 128) >= 64)
-			cfg = 4;
 		else
-			cfg = 2;
+			cfg = 4;
 	}
 	/* the S3K_EPI_QKV epilogue exists for the pipelined kernel with wave
 	 * tiles of 64 columns or 128: the small problems take its 128x128
@@ -990,6 +1000,7 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 	case 2:  return launch_dl_cfg<64, 64, 32, 2, 2, 3, 2, true>(g, p, st);
 	case 3:  return launch_dl_cfg<128, 256, 32, 2, 2, 3, 2>(g, p, st);
 	case 4:  return launch_dl_cfg<128, 128, 64, 2, 2, 2, 2, true>(g, p, st);
+	case 5:  return launch_dl_cfg<64, 64, 64, 2, 2, 4, 2, true>(g, p, st);
 	case 6:  return launch_dl_cfg<192, 256, 32, 2, 2, 4, 1>(g, p, st);
 	case 7:  return launch_dl_cfg<192, 256, 64, 2, 4, 2, 1>(g, p, st);
 	case 8:  return launch_dl_cfg<256, 256, 32, 2, 4, 3, 1>(g, p, st);
@@ -998,6 +1009,7 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 	case 11: return launch_dl_cfg<256, 128, 64, 2, 4, 2, 1>(g, p, st);
 	case 12: return launch_dl_cfg<128, 256, 64, 2, 4, 2, 1>(g, p, st);
 	case 13: return launch_dl_cfg<256, 256, 32, 2, 4, 4, 1>(g, p, st);
+	case 14: return launch_dl_cfg<64, 64, 64, 2, 2, 3, 3, true>(g, p, st);
 	case 20: return launch_dlp_cfg<256, 256, 2, 4, false>(g, p, st);
 	case 21: return launch_dlp_cfg<256, 256, 2, 4, true>(g, p, st);
 	case 22: return launch_dlp_cfg<192, 256, 2, 4, true>(g, p, st);

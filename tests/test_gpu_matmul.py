@@ -320,6 +320,31 @@ def test_dl_pipelined_every_tile_config(env, cfg, K):
     assert_f32_close(c32, ref.astype(np.float32), what=f"dlp cfg {cfg} f16 K={K}")
 
 
+@pytest.mark.parametrize("cfg", [5, 14])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 8), (65, 63 * 8, 72), (129, 200, 192), (200, 520, 264),
+                                   (64, 64, 1544)])
+def test_dl_deep_ring_tiles(env, cfg, M, N, K):
+    """The 64x64 tiles with three or four LDS stages (problems of up to
+    768 such tiles) on fewer k-steps than stages, k tails, ragged rows and
+    columns: against float64, with the bits of the two-stage 128x128 tiles
+    (the same sums in the same order)."""
+    O = oracle()
+    a = O.f32_to_fp16(rnd(218, (M, K))).reshape(M, K)
+    w = O.f32_to_fp16(rnd(219, (N, K), 0.05)).reshape(N, K)
+    bias = O.f32_to_fp16(rnd(220, N, 0.1))
+    out = {}
+    for c in (cfg, 4, -1):
+        env.set("SAM3_HIP_DL_CFG", str(c))
+        out[c] = hip.matmul(a, abi.F16, w, abi.F16, abi.F16, M, N, K, bias=bias,
+                            flags=hip.B_NT | hip.BIAS)
+    assert np.array_equal(out[cfg], out[4]) and np.array_equal(out[-1], out[4])
+    ref = (O.fp16_to_f32(a).reshape(M, K).astype(np.float64) @
+           O.fp16_to_f32(w).reshape(N, K).astype(np.float64).T) + O.fp16_to_f32(bias)
+    # two roundings to f16 (product, then sum): 2 * 2^-11 of the largest value met
+    err = np.abs(O.fp16_to_f32(out[cfg]).reshape(M, N) - ref)
+    assert err.max() <= 2.0 ** -10 * max(1.0, np.abs(ref).max())
+
+
 def test_bf16_output_f32():
     """bf16 operands with an f32 output (no rounding of C)."""
     O = oracle()
