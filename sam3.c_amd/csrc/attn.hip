@@ -174,13 +174,69 @@ struct at_int {
 	static constexpr int value = N;
 };
 
-/* The probabilities of a tile are formed against the running max m
- * without first taking the tile's max: they are only recomputed (after
- * moving m to the tile's max and rescaling the accumulators) when some
+/* The probabilities of half a tile are formed against the running max m
+ * without first taking the half's max: they are only recomputed (after
+ * moving m to the half's max and rescaling the accumulators) when some
  * lane's 32 probabilities sum past 2^15, which also catches the first
  * tile (m = -FLT_MAX gives +inf). Every probability the MFMA sees is
  * then below 2^15, inside the f16 range. */
 constexpr float AT_PSUM_MAX = 32768.0f;
+
+/* Normalize (a query with no finite score keeps zeros, as the reference's
+ * row_sum > 0 test leaves it) and store out[q][d] from a wave's O^T. */
+template <int DT>
+__device__ __forceinline__ void at_store(const AttnArgs &p, const s3k_f32x16 (&o)[2], float l_run,
+					 long long head, int q, int h)
+{
+	const float l_tot = at_sum_pair(l_run);
+	const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+	if (q < p.Sq) {
+#pragma unroll
+		for (int md = 0; md < 2; ++md)
+#pragma unroll
+			for (int g = 0; g < 4; ++g) {
+				const int d0 = 32 * md + 8 * g + 4 * h;
+				const float x0 = o[md][4 * g] * inv, x1 = o[md][4 * g + 1] * inv;
+				const float x2 = o[md][4 * g + 2] * inv, x3 = o[md][4 * g + 3] * inv;
+				const long long orow = at_out_row(p.oh, head, p.Sq, q, AT_D);
+				if constexpr (DT == S3K_F32) {
+					if (p.ofmt == 1) {
+						/* the merged row r = orow / K as bf16 planes,
+						 * the split of split3 / the permute kernel */
+						const long long K = (long long)p.oh * AT_D, r = orow / K;
+						uint16_t *dp = (uint16_t *)p.out + r * 3 * K + (orow - r * K) + d0;
+						uint32_t hi[2], lo[2];
+						split_bf16x2(x0, x1, hi[0], lo[0]);
+						split_bf16x2(x2, x3, hi[1], lo[1]);
+						*(uint2 *)dp = make_uint2(hi[0], hi[1]);
+						*(uint2 *)(dp + K) = make_uint2(lo[0], lo[1]);
+						*(uint2 *)(dp + 2 * K) = make_uint2(hi[0], hi[1]);
+					} else if (p.ofmt == 2) {
+						/* f16, flagged as the permute kernel flags it: a
+						 * value past 2^15, or four nonzero values all
+						 * below 2^-10 */
+						const float ax = __builtin_fabsf(x0), ay = __builtin_fabsf(x1);
+						const float az = __builtin_fabsf(x2), aw = __builtin_fabsf(x3);
+						const float mx = fmaxf(fmaxf(ax, ay), fmaxf(az, aw));
+						const bool big = (ax >= 32768.0f && ax <= 3.402823466e38f) ||
+								 (ay >= 32768.0f && ay <= 3.402823466e38f) ||
+								 (az >= 32768.0f && az <= 3.402823466e38f) ||
+								 (aw >= 32768.0f && aw <= 3.402823466e38f);
+						if (p.ovf && (big || (mx > 0.0f && mx < 0x1p-10f)))
+							*p.ovf = p.ovf_tag;
+						*(uint2 *)((uint16_t *)p.out + orow + d0) =
+							make_uint2(pack_f16x2(x0, x1), pack_f16x2(x2, x3));
+					} else {
+						float *O = (float *)p.out + orow;
+						*(float4 *)(O + d0) = make_float4(x0, x1, x2, x3);
+					}
+				} else {
+					uint16_t *O = (uint16_t *)p.out + orow;
+					*(uint2 *)(O + d0) = make_uint2(at_pack2<DT>(x0, x1), at_pack2<DT>(x2, x3));
+				}
+			}
+	}
+}
 
 template <int DT, int NW, bool MASK, bool VD>
 __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_fwd(AttnArgs p)
@@ -530,15 +586,13 @@ __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_f
 				return ts;
 			};
 			/* if some lane's sum passed the bound: move the max to the
-			 * tile's, rescale what is accumulated, redo half mb (rare) */
+			 * half's, rescale what is accumulated, redo half mb (rare) */
 			auto settle = [&](int mb, float ts) {
 				if (__builtin_amdgcn_ballot_w64(!(ts <= AT_PSUM_MAX))) {
-					float mt = s[0][0];
+					float mt = s[mb][0];
 #pragma unroll
-					for (int b = 0; b < 2; ++b)
-#pragma unroll
-						for (int r = 0; r < 16; ++r)
-							mt = fmaxf(mt, s[b][r]);
+					for (int r = 1; r < 16; ++r)
+						mt = fmaxf(mt, s[mb][r]);
 					const float m_new = fmaxf(m_run, at_max_pair(mt) * LOG2E);
 					const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 					m_run = m_new;
@@ -613,56 +667,374 @@ __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_f
 			step(at_int<1>{}, kt + 1);
 	}
 
-	/* normalize (a query with no finite score keeps zeros, as the
-	 * reference's row_sum > 0 test leaves it) and store out[q][d] */
-	const float l_tot = at_sum_pair(l_run);
-	const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
-	if (q < p.Sq) {
+	at_store<DT>(p, o, l_run, head, q, h);
+}
+
+/* ------------------------------------------------------------------ */
+/* f32 over prepared K and V planes                                     */
+/* ------------------------------------------------------------------ */
+/* attn_fwd splits each f32 K and V tile into bf16 planes while it stages
+ * it, once per block of 128 queries: 81 keys' tiles x 41 query blocks for
+ * a head of 5184 tokens, about as many VALU instructions per tile as the
+ * softmax needs, 32 staging registers, and tiles that cannot arrive by
+ * direct-to-LDS loads. Here the planes are prepared: a K or V row is 256
+ * bytes, hi[64] then lo[64] in bf16 (the bytes of the f32 row it replaces),
+ * written once by attn_planes_k or by the producer of K and V.
+ * The arithmetic per tile is attn_fwd's.
+ *   - Loads: K in two LDS slots, V in one (48 KiB, 168 registers: three
+ *     workgroups per CU), all by direct-to-LDS loads. At the top of a tile
+ *     V of this tile and K of the next are issued; V is waited for, with a
+ *     second barrier, when the scores are done.
+ *   - KS key groups of four waves work on tiles kt = g mod KS of the same
+ *     128 queries and merge through LDS at the end: problems with fewer
+ *     query blocks than CUs keep more than one wave per SIMD.
+ *   - A mask tile (32 queries x 64 keys per wave) is loaded row by row with
+ *     4-byte direct-to-LDS loads (a row of 64 keys is one instruction; any
+ *     row pitch), its 16-byte chunks XOR-swizzled by row, one tile ahead:
+ *     per-lane loads would touch 32 rows, i.e. 32 cache lines, with each
+ *     instruction.
+ * Bound by the MFMAs and the softmax's VALU work on the busiest CUs: 16 x
+ * 5184 x 5184 318 us against 400 for attn_fwd (1038 TFLOP/s of bf16 MFMA;
+ * counters: MFMA busy 52 %, VALU 40 % of the time, 656 workgroups on 768
+ * places), 144 heads x 576 44.7 against 55.2, masked 16 x 1369 47 against
+ * 120. Registers matter: the order of finish_half(1) and settle(0) below
+ * decides whether the kernel spills at 168 (then 155 us where it takes
+ * 105). */
+constexpr int AP_TILE = 2 * AT_K_BYTES;              /* hi and lo, 16 KiB */
+constexpr int AP_GROUP = 3 * AP_TILE;                /* K, K, V */
+constexpr int AP_MASK = 32 * AT_BKV * 4;             /* one wave's mask tile */
+
+/* one dword per lane from global into LDS at lds_addr + 4 * lane */
+__device__ __forceinline__ void dma4s(unsigned lds_addr, s3k_i32x4 rsrc, unsigned voff, unsigned soff)
+{
+	asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tbuffer_load_dword %1, %2, %3 offen lds"
+		     :: "s"(lds_addr), "v"(voff), "s"(rsrc), "s"(soff) : "memory");
+}
+
+template <int KS, bool MASK>
+constexpr int ap_lds()
+{
+	return KS * (AP_GROUP + (MASK ? 4 * AP_MASK : 0));
+}
+
+template <int KS, bool MASK>
+__global__ void __launch_bounds__(256 * KS, KS > 1 ? 1 : MASK ? 2 : 3) attn_planes_fwd(AttnArgs p)
+{
+	__shared__ __attribute__((aligned(1024))) char smem[ap_lds<KS, MASK>()];
+	const int lane = threadIdx.x & 63;
+	const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+	const int grp = KS > 1 ? wave >> 2 : 0, w4 = wave & 3;
+	const int h = lane >> 5, l32 = lane & 31;
+
+	/* workgroup -> (head, query block) as in attn_fwd */
+	const unsigned L = blockIdx.x, nqb = (unsigned)p.nqb;
+	const unsigned g8 = (unsigned)(p.BH / 8) * 8u * nqb;
+	unsigned hh, qb;
+	if (L < g8) {
+		const unsigned sl = L >> 3;
+		hh = sl / nqb * 8u + (L & 7u);
+		qb = sl % nqb;
+	} else {
+		hh = (unsigned)(p.BH / 8) * 8u + (L - g8) / nqb;
+		qb = (L - g8) % nqb;
+	}
+	const long long head = hh;
+	const int q0w = (int)qb * 128 + w4 * 32;
+	const int q = q0w + l32;
+	const bool wave_live = q0w < p.Sq;
+	const unsigned lds0 = lds_addr_of(smem);
+	const unsigned kv0 = (unsigned)grp * AP_GROUP; /* this group's K, K, V slots */
+	constexpr unsigned V0 = 2 * AP_TILE;
+	const unsigned mk0 = (unsigned)(KS * AP_GROUP + wave * AP_MASK);
+
+	uint4 qh[4], ql[4];
+#pragma unroll
+	for (int c = 0; c < 4; ++c) {
+		qh[c] = ql[c] = make_uint4(0, 0, 0, 0);
+		if (q < p.Sq) {
+			const float *Q = (const float *)p.q + head * p.hq + (long long)q * AT_D + 16 * c + 8 * h;
+			float4 x = *(const float4 *)Q, y = *(const float4 *)(Q + 4);
+			x.x *= 0.125f, x.y *= 0.125f, x.z *= 0.125f, x.w *= 0.125f;
+			y.x *= 0.125f, y.y *= 0.125f, y.z *= 0.125f, y.w *= 0.125f;
+			at_split8(x, y, qh[c], ql[c]);
+		}
+	}
+
+	/* rows past Sk read as zeros (offset past the buffer) */
+	const unsigned kv_bytes = (unsigned)((long long)p.Sk * AT_D * 4);
+	const s3k_i32x4 rk = buf_rsrc(p.k + head * p.hk * 4, kv_bytes);
+	const s3k_i32x4 rv = buf_rsrc(p.v + head * p.hk * 4, kv_bytes);
+	constexpr unsigned TILE_BYTES = AT_BKV * AT_D * 4;
+
+	/* a tile is 16 instructions of 1 KiB, four per wave: instruction
+	 * w4 + 4t fills rows 8 ((w4 + 4t) % 8).. of plane (w4 + 4t) / 8; slot s
+	 * of it holds row s / 8, chunk (s % 8) ^ swizzle(row) */
+	unsigned k_off[4], v_off[4];
+#pragma unroll
+	for (int t = 0; t < 4; ++t) {
+		const int j = w4 + 4 * t, s = (j & 7) * 64 + lane, row = s / 8, pl = j >> 3;
+		k_off[t] = (unsigned)(row * 256 + pl * 128 + ((s % 8) ^ lds_swz<8>(row)) * 16);
+		v_off[t] = (unsigned)(row * 256 + pl * 128 + ((s % 8) ^ at_vswz(row)) * 16);
+	}
+	auto issue = [&](int kt, unsigned slot, s3k_i32x4 r, const unsigned (&off)[4]) {
+		const int rows_left = p.Sk - kt * AT_BKV;
+#pragma unroll
+		for (int t = 0; t < 4; ++t) {
+			const int j = w4 + 4 * t, row = ((j & 7) * 64 + lane) / 8;
+			dma16s(lds0 + slot + (unsigned)j * 1024u, r, row < rows_left ? off[t] : S3K_OOB,
+			       (unsigned)kt * TILE_BYTES);
+		}
+	};
+	/* mask rows q0w + r, keys of tile kt: LDS row r, slot s holds the
+	 * 16-byte chunk s ^ (r & 15). Keys past Sk read the next row (or, past
+	 * the mask's end, zeros): their scores become -inf anyway. Rows past Sq
+	 * are past the end. */
+	const s3k_i32x4 rm = MASK ? buf_rsrc(p.mask, (unsigned)((long long)p.Sq * p.Sk * 4)) : rk;
+	auto issue_mask = [&](int kt) {
+#pragma unroll
+		for (int r = 0; r < 32; ++r) {
+			const int row = q0w + r < p.Sq ? q0w + r : p.Sq - 1;
+			dma4s(lds0 + mk0 + (unsigned)r * 256u, rm, (unsigned)((lane ^ ((r & 15) << 2)) << 2),
+			      (unsigned)(((long long)row * p.Sk + kt * AT_BKV) * 4));
+		}
+	};
+
+	unsigned ka[4][2];
+#pragma unroll
+	for (int c = 0; c < 4; ++c)
+#pragma unroll
+		for (int mb = 0; mb < 2; ++mb) {
+			const int row = 32 * mb + l32;
+			ka[c][mb] = kv0 + (unsigned)((row * 8 + ((2 * c + h) ^ lds_swz<8>(row))) << 4);
+		}
+	unsigned vtr[2][2];
+	{
+		const int G = lane >> 4, q16 = lane & 15;
 #pragma unroll
 		for (int md = 0; md < 2; ++md)
 #pragma unroll
-			for (int g = 0; g < 4; ++g) {
-				const int d0 = 32 * md + 8 * g + 4 * h;
-				const float x0 = o[md][4 * g] * inv, x1 = o[md][4 * g + 1] * inv;
-				const float x2 = o[md][4 * g + 2] * inv, x3 = o[md][4 * g + 3] * inv;
-				const long long orow = at_out_row(p.oh, head, p.Sq, q, AT_D);
-				if constexpr (C::SPLIT) {
-					if (p.ofmt == 1) {
-						/* the merged row r = orow / K as bf16 planes,
-						 * the split of split3 / the permute kernel */
-						const long long K = (long long)p.oh * AT_D, r = orow / K;
-						uint16_t *dp = (uint16_t *)p.out + r * 3 * K + (orow - r * K) + d0;
-						uint32_t hi[2], lo[2];
-						split_bf16x2(x0, x1, hi[0], lo[0]);
-						split_bf16x2(x2, x3, hi[1], lo[1]);
-						*(uint2 *)dp = make_uint2(hi[0], hi[1]);
-						*(uint2 *)(dp + K) = make_uint2(lo[0], lo[1]);
-						*(uint2 *)(dp + 2 * K) = make_uint2(hi[0], hi[1]);
-					} else if (p.ofmt == 2) {
-						/* f16, flagged as the permute kernel flags it: a
-						 * value past 2^15, or four nonzero values all
-						 * below 2^-10 */
-						const float ax = __builtin_fabsf(x0), ay = __builtin_fabsf(x1);
-						const float az = __builtin_fabsf(x2), aw = __builtin_fabsf(x3);
-						const float mx = fmaxf(fmaxf(ax, ay), fmaxf(az, aw));
-						const bool big = (ax >= 32768.0f && ax <= 3.402823466e38f) ||
-								 (ay >= 32768.0f && ay <= 3.402823466e38f) ||
-								 (az >= 32768.0f && az <= 3.402823466e38f) ||
-								 (aw >= 32768.0f && aw <= 3.402823466e38f);
-						if (p.ovf && (big || (mx > 0.0f && mx < 0x1p-10f)))
-							*p.ovf = p.ovf_tag;
-						*(uint2 *)((uint16_t *)p.out + orow + d0) =
-							make_uint2(pack_f16x2(x0, x1), pack_f16x2(x2, x3));
-					} else {
-						float *O = (float *)p.out + orow;
-						*(float4 *)(O + d0) = make_float4(x0, x1, x2, x3);
-					}
-				} else {
-					uint16_t *O = (uint16_t *)p.out + orow;
-					*(uint2 *)(O + d0) = make_uint2(at_pack2<DT>(x0, x1), at_pack2<DT>(x2, x3));
-				}
+			for (int hl = 0; hl < 2; ++hl) {
+				const int key = 4 * (G >> 1) + (q16 >> 2) + 8 * hl;
+				const int d = 32 * md + 16 * (G & 1) + 4 * (q16 & 3);
+				vtr[md][hl] = kv0 + V0 +
+					      (unsigned)(key * AT_D * 2 + (((d >> 3) ^ at_vswz(key)) << 4) +
+							 ((d >> 2) & 1) * 8);
 			}
 	}
+
+	s3k_f32x16 o[2];
+#pragma unroll
+	for (int md = 0; md < 2; ++md)
+#pragma unroll
+		for (int r = 0; r < 16; ++r)
+			o[md][r] = 0.0f;
+	float m_run = -3.402823466e38f, l_run = 0.0f;
+	constexpr float LOG2E = 1.44269504088896341f;
+	const int nkt = (p.Sk + AT_BKV - 1) / AT_BKV;
+
+	auto step = [&](auto par, int kt) {
+		constexpr int P = decltype(par)::value;
+		constexpr unsigned KSLOT = P * AP_TILE, KNEXT = (1 - P) * AP_TILE;
+		const bool live = KS == 1 || kt < nkt, more = kt + KS < nkt;
+		/* K(kt) (and the mask tile) landed; every wave is past its last
+		 * reads of the V slot and of the K slot refilled below */
+		wait_vm<0>();
+		wg_barrier();
+		if (live)
+			issue(kt, kv0 + V0, rv, v_off);
+		if (more)
+			issue(kt + KS, kv0 + KNEXT, rk, k_off);
+
+		const int kbase = kt * AT_BKV;
+		s3k_f32x16 s[2];
+		uint4 ph[4], pl[4];
+		float ts0 = 0.0f;
+		auto scores_half = [&](int mb) {
+#pragma unroll
+			for (int r = 0; r < 16; ++r)
+				s[mb][r] = 0.0f;
+#pragma unroll
+			for (int c = 0; c < 4; ++c) {
+				const uint4 kh = *(const uint4 *)(smem + ka[c][mb] + KSLOT);
+				const uint4 kl = *(const uint4 *)(smem + ka[c][mb] + KSLOT + AT_K_BYTES);
+				mfma_chunk<FAM_BF16>(s[mb], kl, qh[c]);
+				mfma_chunk<FAM_BF16>(s[mb], kh, ql[c]);
+				mfma_chunk<FAM_BF16>(s[mb], kh, qh[c]);
+			}
+		};
+		auto finish_half = [&](int mb) {
+			if constexpr (MASK) {
+#pragma unroll
+				for (int g = 0; g < 4; ++g) {
+					const int c = 8 * mb + 2 * g + h; /* chunk of keys 32mb + 8g + 4h.. */
+					const float4 m = *(const float4 *)(smem + mk0 + l32 * 256 +
+									   ((c ^ (l32 & 15)) << 4));
+					s[mb][4 * g] += m.x, s[mb][4 * g + 1] += m.y;
+					s[mb][4 * g + 2] += m.z, s[mb][4 * g + 3] += m.w;
+				}
+			}
+			if (kbase + AT_BKV > p.Sk) {
+#pragma unroll
+				for (int r = 0; r < 16; ++r)
+					if (kbase + 32 * mb + 8 * (r >> 2) + 4 * h + (r & 3) >= p.Sk)
+						s[mb][r] = -__builtin_inff();
+			}
+		};
+		auto probs = [&](int mb) {
+			const float nm = -m_run;
+			float ts = 0.0f;
+#pragma unroll
+			for (int sub = 0; sub < 2; ++sub) {
+				float pv[8];
+#pragma unroll
+				for (int e = 0; e < 8; ++e)
+					pv[e] = __builtin_amdgcn_exp2f(fmaf(s[mb][8 * sub + e], LOG2E, nm));
+				const int cc = 2 * mb + sub;
+#pragma unroll
+				for (int e = 0; e < 8; ++e)
+					ts += pv[e];
+				at_split8(make_float4(pv[0], pv[1], pv[2], pv[3]),
+					  make_float4(pv[4], pv[5], pv[6], pv[7]), ph[cc], pl[cc]);
+			}
+			return ts;
+		};
+		/* as attn_fwd: when some lane's sum passed the bound, move the max
+		 * to the half's, rescale, redo half mb */
+		auto settle = [&](int mb, float ts) {
+			if (__builtin_amdgcn_ballot_w64(!(ts <= AT_PSUM_MAX))) {
+				float mt = s[mb][0];
+#pragma unroll
+				for (int r = 1; r < 16; ++r)
+					mt = fmaxf(mt, s[mb][r]);
+				const float m_new = fmaxf(m_run, at_max_pair(mt) * LOG2E);
+				const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+				m_run = m_new;
+				l_run *= alpha;
+#pragma unroll
+				for (int md = 0; md < 2; ++md)
+#pragma unroll
+					for (int r = 0; r < 16; ++r)
+						o[md][r] *= alpha;
+				ts = probs(mb);
+			}
+			l_run += ts;
+		};
+		auto pv_half = [&](int mb) {
+#pragma unroll
+			for (int md = 0; md < 2; ++md)
+#pragma unroll
+				for (int cc = 2 * mb; cc < 2 * mb + 2; ++cc) {
+					const uint2 hlo = at_read_tr(smem, vtr[md][0] + cc * 2048);
+					const uint2 hhi = at_read_tr(smem, vtr[md][1] + cc * 2048);
+					const uint2 llo = at_read_tr(smem, vtr[md][0] + cc * 2048 + AT_K_BYTES);
+					const uint2 lhi = at_read_tr(smem, vtr[md][1] + cc * 2048 + AT_K_BYTES);
+					const uint4 vh = make_uint4(hlo.x, hlo.y, hhi.x, hhi.y);
+					mfma_chunk<FAM_BF16>(o[md], make_uint4(llo.x, llo.y, lhi.x, lhi.y), ph[cc]);
+					mfma_chunk<FAM_BF16>(o[md], vh, pl[cc]);
+					mfma_chunk<FAM_BF16>(o[md], vh, ph[cc]);
+				}
+		};
+		const bool work = wave_live && live;
+		if (work) {
+			scores_half(0);
+			finish_half(0);
+			scores_half(1);
+			/* (finish before settle: the other order spills registers) */
+			ts0 = probs(0);
+			finish_half(1);
+			settle(0, ts0);
+		}
+		/* V(kt) has landed in every wave's part; K(kt + KS) may still be
+		 * on its way (issued after V) */
+		if (more)
+			wait_vm<4>();
+		else
+			wait_vm<0>();
+		wg_barrier();
+		if constexpr (MASK) {
+			/* this wave has read its mask tile (finish_half(1)) */
+			__builtin_amdgcn_s_waitcnt(0xC07F); /* lgkmcnt(0) */
+			if (wave_live && more)
+				issue_mask(kt + KS);
+		}
+		if (work) {
+			pv_half(0);
+			const float ts1 = probs(1);
+			settle(1, ts1);
+			pv_half(1);
+		}
+	};
+
+	if (grp < nkt) {
+		issue(grp, kv0, rk, k_off);
+		if (MASK && wave_live)
+			issue_mask(grp);
+	}
+	/* every wave runs the same number of steps (the barriers are
+	 * workgroup-wide); a group without a tile left only meets them */
+	const int steps = (nkt + KS - 1) / KS;
+	for (int it = 0; it < steps; it += 2) {
+		step(at_int<0>{}, it * KS + grp);
+		if (it + 1 < steps)
+			step(at_int<1>{}, (it + 1) * KS + grp);
+	}
+
+	if constexpr (KS > 1) {
+		/* merge: the groups g > 0 leave their 34 floats per lane in LDS
+		 * ([value][lane], one 8.5 KiB region per wave, in the K slots no
+		 * wave reads any more), group 0 adds them in order */
+		__syncthreads();
+		constexpr int REG = 34 * 64 * 4;
+		static_assert((KS - 1) * 4 * REG <= KS * AP_GROUP, "merge regions fit");
+		if (grp > 0) {
+			float *r = (float *)(smem + ((grp - 1) * 4 + w4) * REG) + lane;
+			r[0] = m_run;
+			r[64] = l_run;
+#pragma unroll
+			for (int md = 0; md < 2; ++md)
+#pragma unroll
+				for (int e = 0; e < 16; ++e)
+					r[(2 + md * 16 + e) * 64] = o[md][e];
+		}
+		__syncthreads();
+		if (grp > 0)
+			return;
+#pragma unroll
+		for (int g = 1; g < KS; ++g) {
+			const float *r = (const float *)(smem + ((g - 1) * 4 + w4) * REG) + lane;
+			/* the two halves of a query's lanes keep one max (at_max_pair),
+			 * so a group without a finite score has -FLT_MAX, sum 0 */
+			const float m1 = r[0], m = fmaxf(m_run, m1);
+			const float a0 = __builtin_amdgcn_exp2f(m_run - m), a1 = __builtin_amdgcn_exp2f(m1 - m);
+			m_run = m;
+			l_run = l_run * a0 + r[64] * a1;
+#pragma unroll
+			for (int md = 0; md < 2; ++md)
+#pragma unroll
+				for (int e = 0; e < 16; ++e)
+					o[md][e] = o[md][e] * a0 + r[(2 + md * 16 + e) * 64] * a1;
+		}
+	}
+	at_store<S3K_F32>(p, o, l_run, head, q, h);
+}
+
+/* K and V rows (f32, 64 values) -> hi[64] | lo[64] bf16 rows of the same
+ * size; one thread per 8 values. */
+__global__ void __launch_bounds__(256) attn_planes_k(const float *__restrict__ k, const float *__restrict__ v,
+						     char *__restrict__ ko, char *__restrict__ vo,
+						     long long chunks)
+{
+	const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+	if (i >= 2 * chunks)
+		return;
+	const bool isv = i >= chunks;
+	const long long c = isv ? i - chunks : i;
+	const float4 *src = (const float4 *)(isv ? v : k) + 2 * c;
+	uint4 hi, lo;
+	at_split8(src[0], src[1], hi, lo);
+	char *d = (isv ? vo : ko) + (c >> 3) * 256 + (c & 7) * 16;
+	*(uint4 *)d = hi;
+	*(uint4 *)(d + 128) = lo;
 }
 
 /* ------------------------------------------------------------------ */
@@ -1002,6 +1374,40 @@ static int attn_kind_ok(int kind)
 	return kind == S3K_F32 || kind == S3K_BF16 || kind == S3K_F16;
 }
 
+/* Key groups per workgroup of attn_planes_fwd. Up to one workgroup of 128
+ * queries per CU the rest of the CU would stay idle, so that workgroup gets
+ * three groups of waves (two with a mask, whose tiles take LDS), if there
+ * are enough key tiles to share out; past that, one group and up to three
+ * workgroups per CU. 16 heads x 1369 queries x 1369 keys (176 workgroups):
+ * 42.2 us with one group, 32.5 with three; masked 63.0 and 46.9 with two;
+ * 16 x 5184 x 5184 (656): 318 and 323. The tiles asked for grow with the
+ * workgroups: 16 x 576 (80 workgroups, 9 tiles) 23 -> 21 us with the pass
+ * that makes the planes, 40 x 576 (200) 24 -> 26. */
+static int ap_groups(int BH, int Sq, int Sk, bool mask)
+{
+	const long long wgs = (long long)BH * ((Sq + 127) / 128), nkt = (Sk + AT_BKV - 1) / AT_BKV;
+	const bool few = wgs <= 256 && nkt >= 8 && nkt * 16 >= wgs;
+	return !few ? 1 : mask ? 2 : 3;
+}
+
+static int launch_planes(AttnArgs p, hipStream_t st)
+{
+	p.nqb = (p.Sq + 127) / 128;
+	const int ks = ap_groups(p.BH, p.Sq, p.Sk, p.mask != nullptr);
+	const dim3 grid((unsigned)((long long)p.nqb * p.BH));
+#define S3K_AP_GO(KS_, M_) hipLaunchKernelGGL((attn_planes_fwd<KS_, M_>), grid, dim3(256 * KS_), 0, st, p)
+	if (p.mask && ks == 2)
+		S3K_AP_GO(2, true);
+	else if (p.mask)
+		S3K_AP_GO(1, true);
+	else if (ks == 3)
+		S3K_AP_GO(3, false);
+	else
+		S3K_AP_GO(1, false);
+#undef S3K_AP_GO
+	return (int)hipGetLastError();
+}
+
 /* Which kernel runs the problem: S3K_ATTN_MFMA, S3K_ATTN_GENERIC or 0. */
 extern "C" int s3k_attn_path(int kind, const void *q, const void *k, const void *v, void *out,
 			     int BH, int Sq, int Sk, int D)
@@ -1065,12 +1471,65 @@ extern "C" int s3k_attn_heads_path(int kind, const void *q, const void *k, const
 	return attn_heads_pick(0, kind, q, k, v, out, BH, Sq, Sk, D, oh, ofmt);
 }
 
+/* attn_planes_fwd reads the mask through one buffer */
+static bool ap_fits(const void *mask, int Sq, int Sk)
+{
+	return !mask || (long long)Sq * Sk * 4 <= 0x7FFFFFF0LL;
+}
+
+extern "C" int s3k_attn_planes_ok(const void *q, const void *k, const void *v, const void *mask,
+				  void *out, int BH, int Sq, int Sk, int D, int oh, int ofmt)
+{
+	return attn_heads_pick(0, S3K_F32, q, k, v, out, BH, Sq, Sk, D, oh, ofmt) == S3K_ATTN_MFMA &&
+	       ap_fits(mask, Sq, Sk);
+}
+
+/* Whether f32 K and V as they are are worth making planes of first. The
+ * pass over them costs their bytes twice (1296 x 576 keys: 115 us; never
+ * under about 3 us); the gain grows with the query blocks that share them,
+ * and with a mask or idle CUs (ap_groups) there is more to gain. One box,
+ * attn_fwd against pass + attn_planes_fwd, heads x queries [x keys]:
+ * 16 x 5184 (41 blocks) 400 -> 334 us, 64 x 1600 (13) 152 -> 154, 100 x
+ * 1024 (8) 102 -> 108, 1296 x 576 (5) 431 -> 466; masked 16 x 1369 120 ->
+ * 52, 200 x 400 98 -> 71, 1296 x 300 x 200 250 -> 184, 400 x 100 x 600 (1)
+ * 72 -> 79, 16 x 256 16.1 -> 17.1. */
+extern "C" size_t s3k_attn_planes_want(int path, int kind, const void *q, const void *k,
+				       const void *v, const void *mask, void *out, int BH, int Sq,
+				       int Sk, int D, int oh, int ofmt)
+{
+	const int use = s3h_settings()->attn_planes;
+	if (kind != S3K_F32 || use == 0 || (path != 0 && path != S3K_ATTN_MFMA) ||
+	    attn_heads_pick(path, kind, q, k, v, out, BH, Sq, Sk, D, oh, ofmt) != S3K_ATTN_MFMA ||
+	    !ap_fits(mask, Sq, Sk))
+		return 0;
+	const int nqb = (Sq + 127) / 128;
+	const long long tiles = (long long)BH * nqb * ((Sk + AT_BKV - 1) / AT_BKV);
+	const bool shared = mask ? nqb >= 2 && tiles >= 256 : nqb >= 16;
+	if (use < 0 && !shared && ap_groups(BH, Sq, Sk, mask != nullptr) == 1)
+		return 0;
+	return (size_t)BH * (size_t)Sk * AT_D * 4 * 2;
+}
+
+/* The planes of K, then those of V, at dst (s3k_attn_planes_want bytes). */
+extern "C" int s3k_attn_planes_make(const void *k, const void *v, void *dst, int BH, int Sk,
+				    void *stream)
+{
+	const long long chunks = (long long)BH * Sk * (AT_D / 8);
+	const long long wgs = (2 * chunks + 255) / 256;
+	if (wgs <= 0 || wgs >= (1LL << 31))
+		return (int)hipErrorInvalidValue;
+	hipLaunchKernelGGL(attn_planes_k, dim3((unsigned)wgs), dim3(256), 0, (hipStream_t)stream,
+			   (const float *)k, (const float *)v, (char *)dst, (char *)dst + chunks * 32,
+			   chunks);
+	return (int)hipGetLastError();
+}
+
 extern "C" int s3k_attn_heads(int path, int kind, const void *q, const void *k, const void *v,
 			      const float *mask, void *out, int BH, int Sq, int Sk, int D, int oh,
-			      int ofmt, unsigned *ovf, unsigned ovf_tag, void *stream)
+			      int ofmt, unsigned *ovf, unsigned ovf_tag, int kvp, void *stream)
 {
 	path = attn_heads_pick(path, kind, q, k, v, out, BH, Sq, Sk, D, oh, ofmt);
-	if (!path)
+	if (!path || (kvp && (path != S3K_ATTN_MFMA || kind != S3K_F32 || !ap_fits(mask, Sq, Sk))))
 		return (int)hipErrorInvalidValue;
 	if (path == S3K_ATTN_SMALL) {
 		AttnGArgs g{};
@@ -1150,6 +1609,8 @@ extern "C" int s3k_attn_heads(int path, int kind, const void *q, const void *k, 
 			hipLaunchKernelGGL((attn_fwd<DT_, NW_, false, VD_>), grid, block, 0, st, p); \
 	} while (0)
 	const bool vd = s3h_settings()->attn_vdma != 0;
+	if (kvp)
+		return launch_planes(p, st);
 	if (kind == S3K_F32)
 		S3K_ATTN_GO(S3K_F32, 4, false);
 	else if (kind == S3K_BF16) {
@@ -1173,10 +1634,4 @@ extern "C" int s3k_attn_heads(int path, int kind, const void *q, const void *k, 
 	}
 #undef S3K_ATTN_GO
 	return (int)hipGetLastError();
-}
-
-extern "C" int s3k_attn(int path, int kind, const void *q, const void *k, const void *v,
-			const float *mask, void *out, int BH, int Sq, int Sk, int D, void *stream)
-{
-	return s3k_attn_heads(path, kind, q, k, v, mask, out, BH, Sq, Sk, D, 0, 0, nullptr, 0, stream);
 }

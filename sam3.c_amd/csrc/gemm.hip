@@ -552,6 +552,7 @@ static GemmArgs make_args(const struct s3k_gemm *g)
 	p.qkv_H = g->qkv_H;
 	p.qkv_dsh = g->qkv_D > 0 ? __builtin_ctz((unsigned)g->qkv_D) : 0;
 	p.qkv_rope = g->qkv_rope;
+	p.qkv_planes = g->qkv_planes;
 	return p;
 }
 
@@ -571,6 +572,8 @@ static bool qkv_ok(const struct s3k_gemm *g, int path)
 		return false;
 	const int E = H * D, n_out = g->N / E;
 	if (g->N % E || n_out < 1 || n_out > 3 || g->qkv_rope < 0 || (g->qkv_rope >> n_out))
+		return false;
+	if (g->qkv_planes && (sk || D != 64 || g->qkv_planes < 0 || (g->qkv_planes >> n_out)))
 		return false;
 	for (int y = 0; y < n_out; ++y)
 		if (!g->qkv_out[y] || ((uintptr_t)g->qkv_out[y] & 15u))

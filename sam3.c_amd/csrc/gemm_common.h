@@ -38,7 +38,7 @@ struct GemmArgs {
 	/* S3K_EPI_QKV (struct s3k_gemm): head size 1 << qkv_dsh */
 	float *qkv_out[3];
 	const float *qkv_cos, *qkv_sin;
-	int qkv_S, qkv_H, qkv_dsh, qkv_rope;
+	int qkv_S, qkv_H, qkv_dsh, qkv_rope, qkv_planes;
 	int tstrip;   /* tile order (tile_of): 0, or N strips of this many tiles */
 	int xwalk;    /* each slice's tiles on one XCD: gemm_dlk 1; gemm_dlt the
 		       * slice count of its grouped 1-D grid; 0 off */
@@ -609,6 +609,7 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 					: nullptr;
 			const long long hsd = (long long)p.qkv_H * S * D;
 			const bool rope = nok && ((p.qkv_rope >> y) & 1);
+			const bool planes = (p.qkv_planes >> y) & 1;
 			/* this lane's rows: m1 + RPI*k for k = 0, 1, ... over the strips;
 			 * (b, sr): the next row to store, st: the next row whose
 			 * tables are loaded (RPI <= S, so one wrap at a time) */
@@ -663,8 +664,21 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 						x[3] = add_rn(mul_rn(u2, ss.y), mul_rn(u3, cc.y));
 					}
 					const int m = m1 + 32 * i + RPI * it;
-					if (m < p.M && nok)
-						*(float4 *)(ob + b * hsd + (long long)sr * D) = make_float4(x[0], x[1], x[2], x[3]);
+					if (m < p.M && nok) {
+						float *o = ob + b * hsd + (long long)sr * D;
+						if (planes) {
+							/* d = r & 63 of hi[64] | lo[64]: byte 2d of
+							 * the row, where f32 d has byte 4d */
+							uint32_t hi[2], lo[2];
+							split_bf16x2(x[0], x[1], hi[0], lo[0]);
+							split_bf16x2(x[2], x[3], hi[1], lo[1]);
+							uint16_t *w = (uint16_t *)(o - (r & (D - 1))) + (r & (D - 1));
+							*(uint2 *)w = make_uint2(hi[0], hi[1]);
+							*(uint2 *)(w + D) = make_uint2(lo[0], lo[1]);
+						} else {
+							*(float4 *)o = make_float4(x[0], x[1], x[2], x[3]);
+						}
+					}
 					sr += RPI;
 					if (sr >= S) {
 						sr -= S;

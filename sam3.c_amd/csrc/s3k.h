@@ -126,10 +126,12 @@ struct s3k_gemm {
 	 * split. When bit y of qkv_rope is set, RoPE is applied to operand y
 	 * after the bias: pairs (d, d + 1), cos / sin tables [qkv_S, qkv_D/2],
 	 * products and sums rounded separately. qkv_D is a power of two
-	 * >= 4, qkv_S >= 32, N = E, 2E or 3E, M a multiple of qkv_S. */
+	 * >= 4, qkv_S >= 32, N = E, 2E or 3E, M a multiple of qkv_S. When
+	 * bit y of qkv_planes is set (qkv_D = 64, not the skinny kernel),
+	 * each row of operand y is stored as planes (s3k_attn_heads, kvp). */
 	float       *qkv_out[3];
 	const float *qkv_cos, *qkv_sin;
-	int          qkv_S, qkv_H, qkv_D, qkv_rope;
+	int          qkv_S, qkv_H, qkv_D, qkv_rope, qkv_planes;
 };
 
 /* Which kernel s3k_gemm_launch would pick (for tests and the bench). */
@@ -209,25 +211,34 @@ int s3k_cast_f16_rows(int kind, const void *src, long long lda, long long sa, vo
 /* Fused attention out = softmax(Q K^T / sqrt(D) + mask) V over BH heads:
  * Q and out [BH, Sq, D], K and V [BH, Sk, D], one dtype (S3K_F32, _BF16,
  * _F16); mask f32 [Sq, Sk] or NULL. s3k_attn_path gives the kernel that
- * runs the problem (0 = none); s3k_attn runs it on `path` (0 = best:
+ * runs the problem (0 = none); s3k_attn_heads runs it on `path` (0 = best:
  * S3K_ATTN_SMALL when it can run the problem with f32 output rows, else
  * that kernel). S3K_ATTN_SMALL: f32, D = 64, 1 <= Sk <= 128, 16-byte
  * aligned tensors, the latency-bound few-keys kernel. */
 enum { S3K_ATTN_MFMA = 1, S3K_ATTN_GENERIC = 3, S3K_ATTN_SMALL = 4 };
 int s3k_attn_path(int kind, const void *q, const void *k, const void *v, void *out,
 		  int BH, int Sq, int Sk, int D);
-int s3k_attn(int path, int kind, const void *q, const void *k, const void *v,
-	     const float *mask, void *out, int BH, int Sq, int Sk, int D, void *stream);
-/* s3k_attn with the heads merged in the output (oh > 0 heads per batch
+/* s3k_attn_heads with the heads merged in the output (oh > 0 heads per batch
  * item, oh | BH): head b*oh + h, query q is stored at row b*Sq + q,
  * columns h*D.., of [BH/oh * Sq, oh*D], the permute (0,2,1,3) of
- * [BH/oh, oh, Sq, D]. oh = 0 is s3k_attn. ofmt (f32 on the MFMA kernel
+ * [BH/oh, oh, Sq, D]. oh = 0 keeps [BH, Sq, D]. ofmt (f32 on the MFMA kernel
  * only): 0 f32 rows, S3K_LN_PLANES bf16 planes [hi|lo|hi] with row pitch
  * 3*oh*D, S3K_LN_F16 f16 rows storing ovf_tag to *ovf (when set) as
- * s3k_permute_to does: the merged rows as a GEMM's operand. */
+ * s3k_permute_to does: the merged rows as a GEMM's operand.
+ * kvp: K and V are prepared planes, each row of 64 f32 values replaced by
+ * 256 bytes of bf16 hi[64] | lo[64], hi = bf16(x), lo = bf16(x - hi);
+ * only where s3k_attn_planes_ok (k, v: 16-byte aligned). */
 int s3k_attn_heads(int path, int kind, const void *q, const void *k, const void *v,
 		   const float *mask, void *out, int BH, int Sq, int Sk, int D, int oh,
-		   int ofmt, unsigned *ovf, unsigned ovf_tag, void *stream);
+		   int ofmt, unsigned *ovf, unsigned ovf_tag, int kvp, void *stream);
+int s3k_attn_planes_ok(const void *q, const void *k, const void *v, const void *mask, void *out,
+		       int BH, int Sq, int Sk, int D, int oh, int ofmt);
+/* Bytes of scratch for the planes of f32 K and V when making them first
+ * is worth it on this path, else 0; and the pass that makes them. */
+size_t s3k_attn_planes_want(int path, int kind, const void *q, const void *k, const void *v,
+			    const void *mask, void *out, int BH, int Sq, int Sk, int D, int oh,
+			    int ofmt);
+int s3k_attn_planes_make(const void *k, const void *v, void *dst, int BH, int Sk, void *stream);
 /* The kernel s3k_attn_heads(0, ...) runs for these arguments (S3K_ATTN_*,
  * 0 when it refuses them). */
 int s3k_attn_heads_path(int kind, const void *q, const void *k, const void *v, void *out, int BH,
@@ -355,6 +366,9 @@ struct s3h_settings {
 	int attn_vdma;                    /* SAM3_HIP_ATTN_VDMA: 16-bit SDPA V tiles by
 					   * direct-to-LDS loads (1, default) or
 					   * through registers (0) */
+	int attn_planes;                  /* SAM3_HIP_ATTN_PLANES: f32 SDPA over
+					   * prepared K and V planes: -1 by size,
+					   * 0 never, 1 wherever it can run     */
 	int sk_mr, sk_nt;                 /* SAM3_HIP_SK_CFG "mr,nt"             */
 	int q8_expand;                    /* SAM3_HIP_Q8_EXPAND: -1 auto, 0, 1   */
 	int q8_f32cast;                   /* SAM3_HIP_Q8_F32CAST                 */

@@ -659,6 +659,42 @@ static int qkv_epilogue_chains(const struct sam3_graph *g, int i, int j,
 	return n;
 }
 
+/* Whether k and v, the second and third attention operands that the qkv
+ * GEMM at node i stores, may be stored as planes (S3H_KV_PLANES): no node
+ * but one f32 SDPA of head size 64 reads their data (under any header),
+ * none writes it before that, and the SDPA's kernel takes planes. dq:
+ * device address of q. */
+static int kv_planes_fit(const struct sam3_graph *g, int i,
+			 const struct qkv_chain *cs, const void *dq, struct use_map *uses)
+{
+	static const char al[16] __attribute__((aligned(16)));
+	const struct s3h_settings *set = s3h_settings();
+	const struct sam3_tensor *qt = cs[0].out, *kt = cs[1].out, *vt = cs[2].out;
+	if (!set->attn_planes || set->readback_all || kt->dtype != SAM3_DTYPE_F32 ||
+	    uses_of(uses, kt) != 1 || uses_of(uses, vt) != 1 || same_data(kt, vt) || same_data(qt, kt) ||
+	    same_data(qt, vt))
+		return 0;
+	const int s = next_reader(g, i + 1, kt);
+	const struct sam3_node *n = s >= 0 ? &g->nodes[s] : NULL;
+	if (!n || n->op != SAM3_OP_SDPA || !s3h_sdpa_node_ok(n) || n->inputs[0] != qt ||
+	    n->inputs[1] != kt || n->inputs[2] != vt || n->params[0] != 64 || qt->n_dims != 4)
+		return 0;
+	const struct sam3_tensor *mask = n->n_inputs > 3 ? n->inputs[3] : NULL;
+	if (mask && (same_data(mask, kt) || same_data(mask, vt)))
+		return 0;
+	for (int m = 0; m < g->n_nodes; m++) {
+		const struct sam3_node *o = &g->nodes[m];
+		for (int r = 0; m > i && m != s && r < o->n_inputs && r < SAM3_NODE_MAX_INPUTS; r++)
+			if (same_data(o->inputs[r], kt) || same_data(o->inputs[r], vt))
+				return 0;
+		if (m > i && m < s && o->output != kt && o->output != vt &&
+		    (same_data(o->output, kt) || same_data(o->output, vt)))
+			return 0;
+	}
+	return s3k_attn_planes_ok(dq, al, al, mask ? al : NULL, (void *)al, qt->dims[0] * qt->dims[1],
+				  qt->dims[2], kt->dims[2], 64, 0, 0);
+}
+
 /* MATMUL at node i, plus the ADD(bias)/GELU nodes folded into it.
  * Returns the number of nodes consumed in *used. */
 static enum sam3_error run_matmul(struct sam3_hip_backend *hb, const struct sam3_graph *g,
@@ -871,7 +907,16 @@ static enum sam3_error run_matmul(struct sam3_hip_backend *hb, const struct sam3
 		const struct sam3_tensor *ct = NULL, *st = NULL;
 		for (int y = 0; y < n_qkv && err == SAM3_OK; y++) {
 			void *dy = NULL;
-			err = dev_out(hb, qcs[y].out, &dy);
+			if (y == 1 && n_qkv == 3 && kv_planes_fit(g, i, qcs, qkv.out[0], uses)) {
+				qkv.planes = 6;
+				if (!s3h_matmul_qkv_ok(a_fmt, a_dt, da, b_dt, db, M, N, K, flags, &qkv))
+					qkv.planes = 0;
+			}
+			if ((qkv.planes >> y) & 1)
+				err = dev_out_fmt(hb, qcs[y].out, s3h_tensor_bytes(qcs[y].out), S3H_KV_PLANES,
+						  &dy, NULL);
+			else
+				err = dev_out(hb, qcs[y].out, &dy);
 			qkv.out[y] = (float *)dy;
 			if (qcs[y].cos_t) {
 				ct = qcs[y].cos_t;
@@ -1556,11 +1601,19 @@ static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_g
 
 /* ADD, GELU, TRANSPOSE, SDPA, LAYERNORM, ROPE, SLICE on device copies of
  * the node's tensors. */
+/* K and V of this SDPA node hold planes (kv_planes_fit) */
+static int kv_in_planes(struct sam3_hip_backend *hb, const struct sam3_node *n)
+{
+	const struct s3h_res *k = n->n_inputs > 2 && n->inputs[1] ? res_find(hb, n->inputs[1]->data) : NULL;
+	return k && k->fmt == S3H_KV_PLANES;
+}
+
 static enum sam3_error run_elementwise(struct sam3_hip_backend *hb, const struct sam3_node *n)
 {
 	struct sam3_tensor tin[SAM3_NODE_MAX_INPUTS], tout;
 	struct sam3_node dn = *n;
 	enum sam3_error err = SAM3_OK;
+	const int kvp = n->op == SAM3_OP_SDPA && kv_in_planes(hb, n);
 	for (int k = 0; k < n->n_inputs && k < SAM3_NODE_MAX_INPUTS; k++) {
 		if (!n->inputs[k])
 			continue;
@@ -1584,7 +1637,7 @@ static enum sam3_error run_elementwise(struct sam3_hip_backend *hb, const struct
 	else if (n->op == SAM3_OP_GELU)
 		err = s3h_gelu(&dn, hb->stream);
 	else if (n->op == SAM3_OP_SDPA)
-		err = sam3_hip_kernel_sdpa(&dn, hb->stream);
+		err = kvp ? s3h_sdpa_planes(&dn, hb->stream) : sam3_hip_kernel_sdpa(&dn, hb->stream);
 	else if (n->op == SAM3_OP_LAYERNORM)
 		err = s3h_layernorm(&dn, hb->stream);
 	else if (n->op == SAM3_OP_ROPE)
@@ -1654,6 +1707,7 @@ static enum sam3_error run_sdpa_merged(struct sam3_hip_backend *hb, const struct
 	struct sam3_tensor tin[SAM3_NODE_MAX_INPUTS];
 	struct sam3_node dn = *n;
 	enum sam3_error err = SAM3_OK;
+	const int kvp = kv_in_planes(hb, n);
 	for (int k = 0; k < n->n_inputs && k < SAM3_NODE_MAX_INPUTS; k++) {
 		if (!n->inputs[k])
 			continue;
@@ -1689,7 +1743,7 @@ static enum sam3_error run_sdpa_merged(struct sam3_hip_backend *hb, const struct
 				  (size_t)s3h_nelems(t->output) * (fmt == S3H_A_PLANES ? 6 : 2), fmt, &dy,
 				  NULL);
 	if (err == SAM3_OK)
-		err = s3h_sdpa_merged(&dn, dy, fmt, hb->ovf, hb->ovf_tag, hb->stream);
+		err = s3h_sdpa_merged(&dn, dy, fmt, hb->ovf, hb->ovf_tag, kvp, hb->stream);
 	if (err == SAM3_OK) {
 		hb->stats.gpu_nodes++;
 		hb->stats.fused_nodes++;

@@ -20,9 +20,12 @@ size_t s3h_tensor_bytes(const struct sam3_tensor *t);
 /* SDPA node on device tensors with its output stored head-merged
  * ([B, Sq, H, D], the TRANSPOSE (0,2,1,3) of the node's output), as f32
  * or as the operand form fmt (S3H_A_PLANES / S3H_A_F16, f32 SDPA with
- * head size 64) of a GEMM reading rows of H*D. */
+ * head size 64) of a GEMM reading rows of H*D. kvp: K and V are planes
+ * (S3H_KV_PLANES). */
 enum sam3_error s3h_sdpa_merged(const struct sam3_node *node, void *out, int fmt, unsigned *ovf,
-				unsigned ovf_tag, void *stream);
+				unsigned ovf_tag, int kvp, void *stream);
+/* sam3_hip_kernel_sdpa with K and V as planes. */
+enum sam3_error s3h_sdpa_planes(const struct sam3_node *node, void *stream);
 
 /* Device-pointer elementwise nodes used by the dispatcher and graph_eval. */
 enum sam3_error s3h_add(const struct sam3_node *node, void *stream);
@@ -85,7 +88,10 @@ enum sam3_error s3h_bias_add(const struct sam3_node *node, void *stream);
  * producing A can write that form directly: S3H_A_PLANES = bf16 [M, 3K]
  * [hi|lo|hi] (the split f32 GEMM), S3H_A_F16 = f16 [M, K] (the Q8 GEMM
  * with f32 activations). s3h_matmul_fmt runs the GEMM on A in that form. */
-enum { S3H_A_PLAIN = 0, S3H_A_PLANES = 1, S3H_A_F16 = 2, S3H_A_LN = 3, S3H_A_ATT1 = 4 };
+enum { S3H_A_PLAIN = 0, S3H_A_PLANES = 1, S3H_A_F16 = 2, S3H_A_LN = 3, S3H_A_ATT1 = 4,
+       S3H_KV_PLANES = 5 };
+/* S3H_KV_PLANES: not a GEMM operand but K or V of an f32 SDPA as prepared
+ * planes (s3k_attn_heads, kvp). */
 /* S3H_A_LN: A is the output of a LayerNorm that did not run; the skinny
  * Q8_0 GEMM normalizes its input rows itself (S3K_A_LN). With this form
  * the `a` argument of the s3h_matmul_* functions points to this host
@@ -140,6 +146,7 @@ struct s3h_qkv {
 	float *out[3];
 	const float *cos_t, *sin_t;
 	int S, H, D, rope;
+	int planes; /* bit y: operand y as S3H_KV_PLANES (D = 64) */
 };
 /* Whether s3h_matmul_qkv can run this GEMM (s3h_matmul_fmt's, f32 out). */
 int s3h_matmul_qkv_ok(int a_fmt, int a_dt, const void *a, int b_dt, const void *b, int M, int N,

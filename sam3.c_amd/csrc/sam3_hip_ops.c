@@ -1197,6 +1197,7 @@ static void fill_qkv(struct s3k_gemm *g, const struct s3h_qkv *q)
 	g->qkv_H = q->H;
 	g->qkv_D = q->D;
 	g->qkv_rope = q->rope;
+	g->qkv_planes = q->planes;
 	g->flags |= S3K_EPI_QKV;
 }
 
@@ -1239,8 +1240,10 @@ int s3h_matmul_qkv_ok(int a_fmt, int a_dt, const void *a, int b_dt, const void *
 	for (int y = 0; y < n_out; y++)
 		if (!q->out[y] || ((uintptr_t)q->out[y] & 15u))
 			return 0;
+	if (q->planes && (q->D != 64 || q->planes < 0 || (q->planes >> n_out)))
+		return 0;
 	if (!q->rope && qkv_skinny(a_fmt, a_dt, a, b_dt, b, M, N, K, flags))
-		return 1;
+		return !q->planes;
 	return !a_folded(a_fmt) && K % 64 == 0 && q->S >= 32 &&
 	       s3h_matmul_out_ok(a_fmt, a_dt, a, b_dt, b, M, N, K, flags, S3H_A_PLAIN);
 }
@@ -1505,6 +1508,41 @@ enum sam3_error sam3_hip_matmul_q8_noalloc(int a_dtype, const void *a, const voi
 /* ------------------------------------------------------------------ */
 /* Attention                                                            */
 /* ------------------------------------------------------------------ */
+/* s3k_attn_heads; f32 K and V go through planes in scratch first where
+ * that is faster. Not while the stream is being captured (the scratch
+ * would have to be allocated there, and kept for the graph), and not when
+ * there is no memory for them. */
+static enum sam3_error run_attn(int path, int kind, const void *q, const void *k, const void *v,
+				const float *mask, void *out, int BH, int Sq, int Sk, int D, int oh,
+				int ofmt, unsigned *ovf, unsigned ovf_tag, const char *what,
+				void *stream)
+{
+	const size_t want = s3k_attn_planes_want(path, kind, q, k, v, mask, out, BH, Sq, Sk, D, oh, ofmt);
+	void *kv = NULL;
+	if (want) {
+		hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+		if (hipStreamIsCapturing((hipStream_t)stream, &cs) != hipSuccess) {
+			(void)hipGetLastError();
+			cs = hipStreamCaptureStatusActive;
+		}
+		if (cs == hipStreamCaptureStatusNone && s3h_scratch_alloc(&kv, want, stream) != SAM3_OK) {
+			(void)hipGetLastError();
+			kv = NULL;
+		}
+	}
+	if (!kv)
+		return s3h_hip(s3k_attn_heads(path, kind, q, k, v, mask, out, BH, Sq, Sk, D, oh, ofmt, ovf,
+					      ovf_tag, 0, stream),
+			       what);
+	enum sam3_error err = s3h_hip(s3k_attn_planes_make(k, v, kv, BH, Sk, stream), what);
+	if (err == SAM3_OK)
+		err = s3h_hip(s3k_attn_heads(path, kind, q, kv, (const char *)kv + want / 2, mask, out, BH,
+					     Sq, Sk, D, oh, ofmt, ovf, ovf_tag, 1, stream),
+			      what);
+	const enum sam3_error ferr = s3h_scratch_free(kv, stream);
+	return err != SAM3_OK ? err : ferr;
+}
+
 enum sam3_error sam3_hip_sdpa_on_path(int path, int dtype, const void *q, const void *k,
 				      const void *v, const float *mask, void *out, int BH,
 				      int Sq, int Sk, int D, void *stream)
@@ -1537,7 +1575,7 @@ enum sam3_error sam3_hip_sdpa_on_path(int path, int dtype, const void *q, const 
 		s3h_error("sdpa: kernel %d cannot run this problem", path);
 		return SAM3_EINVAL;
 	}
-	return s3h_hip(s3k_attn(path, dtype, q, k, v, mask, out, BH, Sq, Sk, D, stream), "sdpa");
+	return run_attn(path, dtype, q, k, v, mask, out, BH, Sq, Sk, D, 0, 0, NULL, 0, "sdpa", stream);
 }
 
 enum sam3_error sam3_hip_sdpa(int dtype, const void *q, const void *k, const void *v,
@@ -2614,7 +2652,7 @@ enum sam3_error sam3_hip_kernel_sdpa(const struct sam3_node *node, void *stream)
  * reading rows of H*D (f32 SDPA on the MFMA kernel). Inputs read from
  * the node's tensors' data (device addresses). */
 enum sam3_error s3h_sdpa_merged(const struct sam3_node *node, void *out, int fmt, unsigned *ovf,
-				unsigned ovf_tag, void *stream)
+				unsigned ovf_tag, int kvp, void *stream)
 {
 	int BH, Sq, Sk, D;
 	enum sam3_error err = sdpa_shape(node, &BH, &Sq, &Sk, &D, 0);
@@ -2637,10 +2675,27 @@ enum sam3_error s3h_sdpa_merged(const struct sam3_node *node, void *out, int fmt
 		s3h_error("sdpa: unknown output form %d", fmt);
 		return SAM3_EINVAL;
 	}
-	return s3h_hip(s3k_attn_heads(0, dt, Q->data, node->inputs[1]->data, node->inputs[2]->data,
-				      M ? (const float *)M->data : NULL, out, BH, Sq, Sk, D,
-				      Q->dims[1], ofmt, ovf, ovf_tag, stream),
-		       "sdpa (heads merged)");
+	const float *mask = M ? (const float *)M->data : NULL;
+	if (!kvp)
+		return run_attn(0, dt, Q->data, node->inputs[1]->data, node->inputs[2]->data, mask, out, BH,
+				Sq, Sk, D, Q->dims[1], ofmt, ovf, ovf_tag, "sdpa (heads merged)", stream);
+	return s3h_hip(s3k_attn_heads(0, dt, Q->data, node->inputs[1]->data, node->inputs[2]->data, mask,
+				      out, BH, Sq, Sk, D, Q->dims[1], ofmt, ovf, ovf_tag, 1, stream),
+		       "sdpa (heads merged, planes)");
+}
+
+enum sam3_error s3h_sdpa_planes(const struct sam3_node *node, void *stream)
+{
+	int BH, Sq, Sk, D;
+	enum sam3_error err = sdpa_shape(node, &BH, &Sq, &Sk, &D, 0);
+	if (err != SAM3_OK)
+		return err;
+	const struct sam3_tensor *M = node->n_inputs > 3 ? node->inputs[3] : NULL;
+	return s3h_hip(s3k_attn_heads(0, node->inputs[0]->dtype, node->inputs[0]->data,
+				      node->inputs[1]->data, node->inputs[2]->data,
+				      M ? (const float *)M->data : NULL, node->output->data, BH, Sq, Sk,
+				      D, 0, 0, NULL, 0, 1, stream),
+		       "sdpa (planes)");
 }
 
 enum sam3_error sam3_hip_dispatch_node(const struct sam3_node *node, void *stream)

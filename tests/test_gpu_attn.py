@@ -367,3 +367,46 @@ def test_sdpa_graph_eval_2d():
         assert_f32_close(got, oracle().sdpa(q, k, v, None, 8), what="graph sdpa")
     finally:
         be.close()
+
+
+# ------------------------------------- f32 over prepared K and V planes
+@pytest.mark.parametrize("masked", [False, True], ids=["nomask", "mask"])
+@pytest.mark.parametrize("BH,Sq,Sk", [(1, 1, 1), (3, 150, 65), (9, 129, 64), (2, 257, 448),
+                                      (2, 31, 449), (3, 130, 640), (1, 200, 1001)])
+def test_sdpa_planes(env, BH, Sq, Sk, masked):
+    """attn_planes_fwd (SAM3_HIP_ATTN_PLANES=1) at the edges of its key
+    tiles, query blocks and key groups (449 keys and up: two or three
+    groups, some with a tile less), against the oracle; with one group the
+    bits of the kernel that splits K and V itself. The mask holds -inf
+    rows, the type's lowest value over whole key tiles, and odd row
+    pitches."""
+    q, k, v = inputs(1200 + Sq + Sk, BH, Sq, Sk, 64)
+    mask = None
+    if masked:
+        mask = synth.randn(1201 + Sk, (Sq, Sk), 2.0)
+        mask[::5, ::3] = -np.inf
+        mask[Sq // 2, :] = -np.inf
+        mask[Sq // 3, : Sk // 2] = -3.4028234e38
+    env.set("SAM3_HIP_ATTN_PLANES", "1")
+    got, ref = run(abi.F32, q, k, v, mask, path=MFMA)
+    check(abi.F32, got, ref, f"planes {BH}x{Sq}x{Sk} {masked}")
+    env.set("SAM3_HIP_ATTN_PLANES", "0")
+    plain, _ = run(abi.F32, q, k, v, mask, path=MFMA)
+    if Sk <= 448:
+        assert np.array_equal(got.view(np.uint32), plain.view(np.uint32))
+
+
+def test_sdpa_planes_nan_and_inf_scores(env):
+    """A NaN or +inf score makes its query NaN, others stay (as the kernel
+    that splits K and V itself does), also when the key groups merge."""
+    BH, Sq, Sk = 2, 70, 640
+    q, k, v = inputs(1290, BH, Sq, Sk, 64)
+    q[0, 3, 5] = np.nan
+    mask = np.zeros((Sq, Sk), np.float32)
+    mask[7, 600] = np.inf
+    outs = {}
+    for use in ("0", "1"):
+        env.set("SAM3_HIP_ATTN_PLANES", use)
+        outs[use], _ = run(abi.F32, q, k, v, mask, path=MFMA)
+    assert np.isnan(outs["1"][0, 3]).all() and np.isnan(outs["1"][:, 7]).all()
+    assert np.array_equal(np.isnan(outs["0"]), np.isnan(outs["1"]))

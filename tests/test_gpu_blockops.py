@@ -998,3 +998,48 @@ def test_vit_block_full_size_global(env, wkind):
     R.close()
     assert_f32_close(y, ref, floor=1.5e-2 if wkind == "q8" else 2e-3,
                      what=f"full-size global block {wkind}")
+
+
+@pytest.mark.parametrize("grid,window,is_global", [(12, 6, False), (18, 9, False), (14, 14, True)])
+@pytest.mark.parametrize("wkind", ["f32", "q8"])
+def test_qkv_gemm_stores_key_and_value_planes(env, wkind, grid, window, is_global):
+    """A ViT block whose qkv GEMM stores K and V as the bf16 planes its
+    attention reads, where the kernel choice allows (36 and 196 keys; 81
+    keys keep the few-keys kernel): the same bits as f32 K and V
+    (SAM3_HIP_ATTN_PLANES=0)."""
+    e, heads, npos = 256, 4, grid * grid
+
+    def run(mode):
+        env.set("SAM3_HIP_ATTN_PLANES", mode)
+        G = graph.Graph()
+        x = G.tensor(abi.F32, (npos, e), synth.randn(1300, (npos, e)), ephemeral=1)
+
+        def w(i, shape, std, quant=False):
+            v = synth.randn(1300 + i, shape, std)
+            if quant and wkind == "q8":
+                return G.tensor(abi.Q8_0, shape, oracle().q8_quantize(v))
+            return G.tensor(abi.F32, shape, v)
+        p = {"ln1_w": w(1, (e,), 1.0), "ln1_b": w(2, (e,), 0.1),
+             "qkv_w": w(3, (3 * e, e), 0.05, True), "qkv_b": w(4, (3 * e,), 0.02),
+             "proj_w": w(5, (e, e), 0.05, True), "proj_b": w(6, (e,), 0.02),
+             "ln2_w": w(7, (e,), 1.0), "ln2_b": w(8, (e,), 0.1),
+             "fc1_w": w(9, (2 * e, e), 0.05, True), "fc1_b": w(10, (2 * e,), 0.02),
+             "fc2_w": w(11, (e, 2 * e), 0.05, True), "fc2_b": w(12, (e,), 0.02)}
+        c, s_ = graph.rope_tables(grid if is_global else window, e // heads)
+        tc, ts = G.tensor(abi.F32, c.shape, c), G.tensor(abi.F32, s_.shape, s_)
+        out = graph.vit_block(G, x, p, heads, grid, window, is_global, tc, ts)
+        be = hip.Backend(0)
+        try:
+            res = []
+            for _ in range(2):  # the second eval reuses the allocations
+                assert be.graph_eval(G.g) == abi.OK
+                assert be.stats().host_nodes == 0
+                res.append(np.ctypeslib.as_array(C.cast(out.data, C.POINTER(C.c_float)),
+                                                 shape=(npos, e)).copy())
+        finally:
+            be.close()
+        assert np.array_equal(res[0], res[1])
+        return res[0]
+
+    a, b = run("-1"), run("0")
+    assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
