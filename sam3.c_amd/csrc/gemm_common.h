@@ -366,6 +366,59 @@ struct epi_b {
 	static constexpr bool value = B;
 };
 
+/* The largest of v over the aligned group of L lanes (L = 4, 8 or 16) that
+ * this lane is in: DPP lane exchanges instead of LDS ones. */
+template <int L>
+__device__ __forceinline__ float group_max(float v)
+{
+	static_assert(L == 4 || L == 8 || L == 16, "DPP row groups");
+#define S3K_DPP_MAX(ctrl) \
+	v = fmaxf(v, __int_as_float(__builtin_amdgcn_mov_dpp(__float_as_int(v), ctrl, 0xF, 0xF, true)))
+	S3K_DPP_MAX(0xB1); /* quad_perm: lane ^ 1 */
+	S3K_DPP_MAX(0x4E); /* quad_perm: lane ^ 2 */
+	if constexpr (L >= 8)
+		S3K_DPP_MAX(0x141); /* row_half_mirror: the other four of eight */
+	if constexpr (L >= 16)
+		S3K_DPP_MAX(0x140); /* row_mirror: the other eight of sixteen */
+#undef S3K_DPP_MAX
+	return v;
+}
+
+/* The output row of row m under the map, then of m + step after each
+ * next(step): out_row without its divisions. */
+struct RowWalk {
+	int g, d1, d2, a, b, c, w, m;
+	__device__ __forceinline__ RowWalk(const GemmArgs &p, int m0)
+		: g(p.rm_g), d1(p.rm_d1), d2(p.rm_d2), a(0), b(0), c(0), w(0), m(m0)
+	{
+		if (g) {
+			const int gi = m0 / g, t = gi / d2;
+			w = m0 - gi * g;
+			c = gi - t * d2;
+			a = t / d1;
+			b = t - a * d1;
+		}
+	}
+	__device__ __forceinline__ long long row() const
+	{
+		return g ? ((long long)(a * d2 + c) * d1 + b) * g + w : m;
+	}
+	__device__ __forceinline__ void next(int step)
+	{
+		m += step;
+		if (!g)
+			return;
+		for (w += step; w >= g; w -= g)
+			if (++c == d2) {
+				c = 0;
+				if (++b == d1) {
+					b = 0;
+					++a;
+				}
+			}
+	}
+};
+
 /* Epilogue of a wave tile, one 32-row strip at a time: the MFMA layout is
  * turned into row-contiguous runs of columns through LDS, so each lane
  * finishes 4 (f32) or 8 (16-bit) outputs and writes them with one 16-byte
@@ -490,9 +543,13 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 	 * arithmetic relies on this path issuing exactly FM * UNITS / 64
 	 * stores per lane and no load for whole tiles (dlk_ok admits only
 	 * problems that take it). */
-	constexpr bool PLAIN_CK = CK == S3K_F32 || CK == S3K_BF16 || CK == S3K_F16;
-	const bool fast = PLAIN_CK && !(flags & S3K_EPI_RES) && (FIXED || !(flags & S3K_EPI_BIAS)) &&
-			  !p.rm_g && p.vec_ok && n0 + WTN <= p.N;
+	constexpr bool OPERAND_CK = CK == S3K_C_PLANES || CK == S3K_C_F16OP;
+	/* the operand kinds take it too: 5184x4096x1024 with bias and GELU to
+	 * an f16 operand with row tags 75.2 -> 65.4 us (the general path below
+	 * spent its time on per-value checks and LDS lane exchanges) */
+	const bool whole = p.vec_ok && n0 + WTN <= p.N;
+	const bool fast = !(flags & S3K_EPI_RES) && (FIXED || !(flags & S3K_EPI_BIAS)) && !p.rm_g &&
+			  whole && (CK != S3K_C_F16OP || FIXED);
 	EpiIn<W> ein;
 #pragma unroll
 	for (int q = 0; q < W; ++q) {
@@ -557,7 +614,46 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 						v[it][e] = epilogue<CK>(v[it][e], ein.b[e], (EB ? S3K_EPI_BIAS : 0) |
 												(EG ? S3K_EPI_GELU : 0));
 				}
-				if (m < p.M) {
+				if constexpr (CK == S3K_C_F16OP && FIXED) {
+					/* the range checks of finishw, on the largest |x| of
+					 * the unit (NaN drops out of it): below 2^15 no value
+					 * is big or infinite and it is the unit's finite
+					 * maximum; other units take the checks per value */
+					float mx = 0.0f;
+#pragma unroll
+					for (int e = 0; e < W; ++e)
+						mx = fmaxf(mx, __builtin_fabsf(v[it][e]));
+					if (!(mx < 32768.0f)) {
+						if (m < p.M && p.ovf && f16_big<W>(v[it]))
+							*p.ovf = p.ovf_tag;
+						mx = f16_part_max<W>(v[it]);
+					}
+					if (p.rowf) {
+						mx = group_max<(WTN / W < 16 ? WTN / W : 16)>(mx);
+						if ((lane & (WTN / W - 1)) == 0 && m < p.M)
+							f16_row_tag(p, m, mx);
+					}
+				}
+				if constexpr (OPERAND_CK) {
+					/* plain stores: the next GEMM reads them at once */
+					if (m < p.M) {
+						uint16_t *c = (uint16_t *)cb + (long long)m * p.ldc + n;
+						uint32_t hi[4], lo[4];
+#pragma unroll
+						for (int e = 0; e < 4; ++e) {
+							const float x0 = v[it][2 * e], x1 = v[it][2 * e + 1];
+							if constexpr (CK == S3K_C_PLANES)
+								split_bf16x2(x0, x1, hi[e], lo[e]);
+							else
+								hi[e] = pack_f16x2(x0, x1);
+						}
+						*(s3k_u32x4 *)c = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
+						if constexpr (CK == S3K_C_PLANES) {
+							*(s3k_u32x4 *)(c + p.N) = (s3k_u32x4){lo[0], lo[1], lo[2], lo[3]};
+							*(s3k_u32x4 *)(c + 2LL * p.N) = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
+						}
+					}
+				} else if (m < p.M) {
 					/* streaming (non-temporal) stores: the tile is
 					 * written once and not read back by this kernel,
 					 * so it need not displace the operand panels
@@ -684,6 +780,62 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 						sr -= S;
 						++b;
 					}
+				}
+				wave_lds_fence();
+			}
+			return;
+		}
+	}
+	/* f32 with a residual, whole tiles: the residual of strip i + 1 is
+	 * loaded before strip i's stores (a load issued after a store waits for
+	 * it), and the row map is walked instead of divided out per store.
+	 * 5184x1024 f32 out on 192x128 tiles: K 1024 with the row map 30.6 ->
+	 * 24.6 us, K 4096 49.4 -> 43.3 (f16 operands) */
+	if constexpr (CK == S3K_F32 && FIXED) {
+		if ((flags & S3K_EPI_RES) && whole && !(flags & S3K_EPI_GELU) && p.ldr % 4 == 0 &&
+		    !((uintptr_t)p.res & 15u)) {
+			constexpr int IT = UNITS / 64, LPR = WTN / W, RPI = 64 / LPR;
+			const bool eb = flags & S3K_EPI_BIAS;
+			const int n = n0 + (lane % LPR) * W;
+			const float *res = (const float *)p.res + n;
+			RowWalk rw(p, m0 + lane / LPR);
+			float4 rb[2][IT];
+			long long ro[2][IT];
+			auto load_res = [&](float4 (&r)[IT], long long (&o)[IT]) {
+#pragma unroll
+				for (int it = 0; it < IT; ++it) {
+					o[it] = rw.m < p.M ? rw.row() : -1;
+					r[it] = make_float4(0.f, 0.f, 0.f, 0.f);
+					if (o[it] >= 0)
+						r[it] = *(const float4 *)(res + o[it] * p.ldr);
+					rw.next(RPI);
+				}
+			};
+			load_res(rb[0], ro[0]);
+#pragma unroll
+			for (int i = 0; i < FM; ++i) {
+				if (i + 1 < FM)
+					load_res(rb[(i + 1) & 1], ro[(i + 1) & 1]);
+				stage(acc[i]);
+				wave_lds_fence();
+				float v[IT][W];
+#pragma unroll
+				for (int it = 0; it < IT; ++it)
+					staged(lane + 64 * it, v[it]);
+#pragma unroll
+				for (int it = 0; it < IT; ++it) {
+					const float4 r = rb[i & 1][it];
+					const float rr[4] = {r.x, r.y, r.z, r.w};
+#pragma unroll
+					for (int e = 0; e < W; ++e) {
+						if (eb)
+							v[it][e] = add_rn(v[it][e], ein.b[e]);
+						v[it][e] = add_rn(v[it][e], rr[e]);
+					}
+					const long long o = ro[i & 1][it];
+					if (o >= 0)
+						*(float4 *)((float *)cb + o * p.ldc + n) =
+							make_float4(v[it][0], v[it][1], v[it][2], v[it][3]);
 				}
 				wave_lds_fence();
 			}

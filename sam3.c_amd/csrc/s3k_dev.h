@@ -246,7 +246,9 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi)
 __device__ __forceinline__ void split_bf16x2(float a, float b, uint32_t &hi, uint32_t &lo)
 {
 	hi = pack_bf16x2(a, b);
-	lo = pack_bf16x2(a - __uint_as_float(hi << 16), b - __uint_as_float(hi & 0xFFFF0000u));
+	/* sub_rn: x - hi of the rounded x, not of the product x may come from */
+	lo = pack_bf16x2(sub_rn(a, __uint_as_float(hi << 16)),
+			 sub_rn(b, __uint_as_float(hi & 0xFFFF0000u)));
 }
 
 __device__ __forceinline__ float round_bf16_hw(float f)

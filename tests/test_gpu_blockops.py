@@ -1007,39 +1007,60 @@ def test_qkv_gemm_stores_key_and_value_planes(env, wkind, grid, window, is_globa
     attention reads, where the kernel choice allows (36 and 196 keys; 81
     keys keep the few-keys kernel): the same bits as f32 K and V
     (SAM3_HIP_ATTN_PLANES=0)."""
-    e, heads, npos = 256, 4, grid * grid
-
     def run(mode):
         env.set("SAM3_HIP_ATTN_PLANES", mode)
-        G = graph.Graph()
-        x = G.tensor(abi.F32, (npos, e), synth.randn(1300, (npos, e)), ephemeral=1)
-
-        def w(i, shape, std, quant=False):
-            v = synth.randn(1300 + i, shape, std)
-            if quant and wkind == "q8":
-                return G.tensor(abi.Q8_0, shape, oracle().q8_quantize(v))
-            return G.tensor(abi.F32, shape, v)
-        p = {"ln1_w": w(1, (e,), 1.0), "ln1_b": w(2, (e,), 0.1),
-             "qkv_w": w(3, (3 * e, e), 0.05, True), "qkv_b": w(4, (3 * e,), 0.02),
-             "proj_w": w(5, (e, e), 0.05, True), "proj_b": w(6, (e,), 0.02),
-             "ln2_w": w(7, (e,), 1.0), "ln2_b": w(8, (e,), 0.1),
-             "fc1_w": w(9, (2 * e, e), 0.05, True), "fc1_b": w(10, (2 * e,), 0.02),
-             "fc2_w": w(11, (e, 2 * e), 0.05, True), "fc2_b": w(12, (e,), 0.02)}
-        c, s_ = graph.rope_tables(grid if is_global else window, e // heads)
-        tc, ts = G.tensor(abi.F32, c.shape, c), G.tensor(abi.F32, s_.shape, s_)
-        out = graph.vit_block(G, x, p, heads, grid, window, is_global, tc, ts)
-        be = hip.Backend(0)
-        try:
-            res = []
-            for _ in range(2):  # the second eval reuses the allocations
-                assert be.graph_eval(G.g) == abi.OK
-                assert be.stats().host_nodes == 0
-                res.append(np.ctypeslib.as_array(C.cast(out.data, C.POINTER(C.c_float)),
-                                                 shape=(npos, e)).copy())
-        finally:
-            be.close()
-        assert np.array_equal(res[0], res[1])
-        return res[0]
+        return small_vit_block(wkind, grid, window, is_global)
 
     a, b = run("-1"), run("0")
     assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+@pytest.mark.parametrize("grid,window", [(9, 3), (15, 5), (18, 9), (64, 8)])
+@pytest.mark.parametrize("wkind", ["f32", "q8"])
+def test_block_epilogues_keep_the_bits_of_separate_nodes(env, wkind, grid, window):
+    """The GEMM epilogues of a windowed block (residual and row map, operand
+    forms) on whole tiles with a ragged M, window sides below, at and above
+    the rows a wave steps by (8), the 64x64 and the 192x128 tiles: the bits
+    of the residual ADD, the unpartition and the conversions as nodes and
+    passes of their own."""
+    def run(mode):
+        for n in ("RESIDUAL_FOLD", "UNPARTITION_FOLD", "GEMM_OPERAND"):
+            env.set("SAM3_HIP_" + n, mode)
+        return small_vit_block(wkind, grid, window, False)
+
+    a, b = run("1"), run("0")
+    assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
+
+
+def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
+    """Output of one ViT block of width e, evaluated twice on one backend."""
+    npos = grid * grid
+    G = graph.Graph()
+    x = G.tensor(abi.F32, (npos, e), synth.randn(1300, (npos, e)), ephemeral=1)
+
+    def w(i, shape, std, quant=False):
+        v = synth.randn(1300 + i, shape, std)
+        if quant and wkind == "q8":
+            return G.tensor(abi.Q8_0, shape, oracle().q8_quantize(v))
+        return G.tensor(abi.F32, shape, v)
+    p = {"ln1_w": w(1, (e,), 1.0), "ln1_b": w(2, (e,), 0.1),
+         "qkv_w": w(3, (3 * e, e), 0.05, True), "qkv_b": w(4, (3 * e,), 0.02),
+         "proj_w": w(5, (e, e), 0.05, True), "proj_b": w(6, (e,), 0.02),
+         "ln2_w": w(7, (e,), 1.0), "ln2_b": w(8, (e,), 0.1),
+         "fc1_w": w(9, (2 * e, e), 0.05, True), "fc1_b": w(10, (2 * e,), 0.02),
+         "fc2_w": w(11, (e, 2 * e), 0.05, True), "fc2_b": w(12, (e,), 0.02)}
+    c, s_ = graph.rope_tables(grid if is_global else window, e // heads)
+    tc, ts = G.tensor(abi.F32, c.shape, c), G.tensor(abi.F32, s_.shape, s_)
+    out = graph.vit_block(G, x, p, heads, grid, window, is_global, tc, ts)
+    be = hip.Backend(0)
+    try:
+        res = []
+        for _ in range(2):  # the second eval reuses the allocations
+            assert be.graph_eval(G.g) == abi.OK
+            assert be.stats().host_nodes == 0
+            res.append(np.ctypeslib.as_array(C.cast(out.data, C.POINTER(C.c_float)),
+                                             shape=(npos, e)).copy())
+    finally:
+        be.close()
+    assert np.array_equal(res[0], res[1])
+    return res[0]
