@@ -364,7 +364,7 @@ __global__ void __launch_bounds__(256, 1) gemm_tiled(GemmArgs p)
 	}
 
 	static_assert(4 * 32 * (WTN + 8) * 4 <= 2 * STAGE, "epilogue staging fits");
-	write_tile_ck<FM, FN, WTN, CK>(p, acc, smem, wave, lane, tm * BM + wm0, tn * BN + wn0, bz);
+	write_tile_ck<FM, FN, WTN, CK, false, false, false>(p, acc, smem, wave, lane, tm * BM + wm0, tn * BN + wn0, bz);
 }
 
 /* ------------------------------------------------------------------ */

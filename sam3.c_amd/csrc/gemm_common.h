@@ -440,9 +440,11 @@ struct RowWalk {
  * once per strip; the residual loop is kept rolled (it loads inside the
  * loop, and unrolled it would not fit the instruction cache), and each of
  * its iterations reads the next iteration's staged values first.
+ * RES_OK false: no unrolled residual path (the kernel's registers leave
+ * no room for it, or it takes no residual).
  * QKV_OK (TR, f32 output): the S3K_EPI_QKV epilogue only, a kernel of
  * its own (the other paths' registers would not leave room for it). */
-template <int FM, int FN, int WTN, int CK, bool TR = false, bool QKV_OK = false>
+template <int FM, int FN, int WTN, int CK, bool TR = false, bool QKV_OK = false, bool RES_OK = true>
 __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&acc)[FM][FN],
 					      char *smem, int wave, int lane, int m0, int n0, int bz)
 {
@@ -791,7 +793,7 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 	 * it), and the row map is walked instead of divided out per store.
 	 * 5184x1024 f32 out on 192x128 tiles: K 1024 with the row map 30.6 ->
 	 * 24.6 us, K 4096 49.4 -> 43.3 (f16 operands) */
-	if constexpr (CK == S3K_F32 && FIXED) {
+	if constexpr (CK == S3K_F32 && FIXED && RES_OK && UNITS / 64 <= 8) {
 		if ((flags & S3K_EPI_RES) && whole && !(flags & S3K_EPI_GELU) && p.ldr % 4 == 0 &&
 		    !((uintptr_t)p.res & 15u)) {
 			constexpr int IT = UNITS / 64, LPR = WTN / W, RPI = 64 / LPR;
@@ -938,7 +940,7 @@ __device__ __forceinline__ void write_tile(const GemmArgs &p, s3k_f32x16 (&acc)[
 					   int wave, int lane, int m0, int n0, int bz)
 {
 	if (p.c_kind == S3K_F32)
-		write_tile_ck<FM, FN, WTN, S3K_F32>(p, acc, smem, wave, lane, m0, n0, bz);
+		write_tile_ck<FM, FN, WTN, S3K_F32, false, false, false>(p, acc, smem, wave, lane, m0, n0, bz);
 	else if (p.c_kind == S3K_BF16)
 		write_tile_ck<FM, FN, WTN, S3K_BF16>(p, acc, smem, wave, lane, m0, n0, bz);
 	else

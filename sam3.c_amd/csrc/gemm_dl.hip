@@ -497,7 +497,7 @@ __global__ void __launch_bounds__(128 * WGN, 1) gemm_dlk(GemmArgs p, int total)
 			load_tile(xw ? tile_at(q + qstep) : q + qstep, b ^ 1);
 		int bz, tm, tn;
 		coords(t, bz, tm, tn);
-		write_tile_ck<FM, FN, WTN, CK, true>(p, acc, smem + 2 * STAGE, wave, lane, tm * BM + wm0,
+		write_tile_ck<FM, FN, WTN, CK, true, false, false>(p, acc, smem + 2 * STAGE, wave, lane, tm * BM + wm0,
 						      tn * BN + wn0, bz);
 	}
 }
