@@ -341,7 +341,9 @@ static int launch_conv_cfg(ConvArgs q, int kind, hipStream_t st)
 	q.g.tiles_m = (q.g.M + BM - 1) / BM;
 	q.g.tiles_n = (q.g.N + BN - 1) / BN;
 	const dim3 grid(q.g.tiles_m * q.g.tiles_n), block(64 * WGM * WGN);
-	if (kind == S3K_F32)
+	if (kind == S3K_F32 && q.g.c_kind == S3K_C_PLANES)
+		hipLaunchKernelGGL((conv_dl<BM, BN, BK, WGM, WGN, STAGES, FAM_BF16, S3K_C_PLANES, OCC>), grid, block, 0, st, q);
+	else if (kind == S3K_F32)
 		hipLaunchKernelGGL((conv_dl<BM, BN, BK, WGM, WGN, STAGES, FAM_BF16, S3K_F32, OCC>), grid, block, 0, st, q);
 	else if (kind == S3K_BF16)
 		hipLaunchKernelGGL((conv_dl<BM, BN, BK, WGM, WGN, STAGES, FAM_BF16, S3K_BF16, OCC>), grid, block, 0, st, q);
@@ -384,9 +386,11 @@ extern "C" int s3k_conv_implicit(const struct s3k_conv *c, const void *xa, const
 	q.g.N = c->OC;
 	q.g.K = K1 * segs;
 	q.g.ldb_b = (long long)K1 * segs * 2;
-	q.g.ldc = c->OC;
+	if (c->out_planes && (c->kind != S3K_F32 || c->OC % 8))
+		return (int)hipErrorInvalidValue;
+	q.g.ldc = c->out_planes ? 3 * c->OC : c->OC;
 	q.g.flags = c->flags & (S3K_EPI_BIAS | S3K_EPI_GELU);
-	q.g.c_kind = c->kind;
+	q.g.c_kind = c->out_planes ? S3K_C_PLANES : c->kind;
 	q.g.bias_kind = c->kind;
 	q.g.vec_ok = (c->OC % 8 == 0) && (((uintptr_t)c->y & 15u) == 0);
 	q.g.a_extent = (unsigned)a_bytes;
@@ -398,15 +402,22 @@ extern "C" int s3k_conv_implicit(const struct s3k_conv *c, const void *xa, const
 	int cfg = s3h_settings()->conv_cfg;
 	/* Tiles (measured on the neck shapes): 64x64 when 128x128 tiles would
 	 * not cover the 256 CUs (72x72 maps: 5184 x 256), else the GEMM's
-	 * rule (256x256 for one nearly full round, 192x128 from 192 tiles). */
+	 * rule (256x256 for one nearly full round, 192x128 from 192 tiles).
+	 * The 64x64 tiles keep three k-steps in flight (four stages, two
+	 * workgroups per CU up to 512 tiles, three stages above): 1x1 over
+	 * 72x72x1024 (k' 3072) 26.6 -> 22.6 us, 3x3 over 72x72x256 47.8 ->
+	 * 45, over 36x36x256 (84 tiles, 108 k-steps) 45 -> 28. */
 	if (cfg < 0) {
 		const long long t9 = conv_tiles(q.g.M, q.g.N, 256, 256), t10 = conv_tiles(q.g.M, q.g.N, 192, 128);
-		cfg = conv_tiles(q.g.M, q.g.N, 128, 128) < 256 ? 2 : (t9 >= 224 && t9 <= 256) ? 9 : t10 >= 192 ? 10 : 4;
+		const long long t6 = conv_tiles(q.g.M, q.g.N, 64, 64);
+		cfg = conv_tiles(q.g.M, q.g.N, 128, 128) < 256 ? (t6 <= 512 ? 6 : 7) : (t9 >= 224 && t9 <= 256) ? 9 : t10 >= 192 ? 10 : 4;
 	}
 	switch (cfg) {
 	case 2:  return launch_conv_cfg<64, 64, 64, 2, 2, 2, 2>(q, c->kind, st);
 	case 4:  return launch_conv_cfg<128, 128, 64, 2, 2, 2, 2>(q, c->kind, st);
 	case 5:  return launch_conv_cfg<128, 64, 64, 2, 2, 2, 2>(q, c->kind, st);
+	case 6:  return launch_conv_cfg<64, 64, 64, 2, 2, 4, 2>(q, c->kind, st);
+	case 7:  return launch_conv_cfg<64, 64, 64, 2, 2, 3, 3>(q, c->kind, st);
 	case 9:  return launch_conv_cfg<256, 256, 64, 2, 4, 2, 1>(q, c->kind, st);
 	case 10: return launch_conv_cfg<192, 128, 64, 2, 4, 2, 1>(q, c->kind, st);
 	default: return (int)hipErrorInvalidValue;

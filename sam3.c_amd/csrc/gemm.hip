@@ -553,6 +553,9 @@ static GemmArgs make_args(const struct s3k_gemm *g)
 	p.qkv_dsh = g->qkv_D > 0 ? __builtin_ctz((unsigned)g->qkv_D) : 0;
 	p.qkv_rope = g->qkv_rope;
 	p.qkv_planes = g->qkv_planes;
+	p.ps_s = g->ps_s;
+	p.ps_oc = g->ps_oc;
+	p.ps_w = g->ps_w;
 	return p;
 }
 
@@ -706,6 +709,14 @@ extern "C" int s3k_gemm_launch_path(const struct s3k_gemm *g, int path, void *st
 	if ((g->flags & S3K_EPI_QKV) &&
 	    ((path != S3K_PATH_MFMA && path != S3K_PATH_SKINNY) ||
 	     (path == S3K_PATH_MFMA && !mfma_ok(g)) || !qkv_ok(g, path)))
+		return (int)hipErrorInvalidValue;
+	/* the pixel shuffle lives in the epilogue's unrolled store path: whole
+	 * wave tiles of columns, 16-byte rows, the direct-to-LDS kernels */
+	if (g->ps_s &&
+	    (g->ps_s < 0 || path != S3K_PATH_MFMA || !s3k_dl_ok(g) || g->batch != 1 || g->rm_g ||
+	     (g->flags & (S3K_EPI_RES | S3K_EPI_QKV)) || g->ps_oc <= 0 || g->ps_oc % 64 ||
+	     (long long)g->ps_s * g->ps_s * g->ps_oc != g->N || g->ps_w <= 0 || g->M % g->ps_w ||
+	     (g->c_kind != S3K_F32 && g->c_kind != S3K_C_PLANES) || !p.vec_ok))
 		return (int)hipErrorInvalidValue;
 	/* the weight-row factors: every MFMA GEMM rounding q*scale to f16
 	 * applies them (S3K_EPI_COLSCALE), and only the MFMA epilogue takes

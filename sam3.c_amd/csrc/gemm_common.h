@@ -39,6 +39,7 @@ struct GemmArgs {
 	float *qkv_out[3];
 	const float *qkv_cos, *qkv_sin;
 	int qkv_S, qkv_H, qkv_dsh, qkv_rope, qkv_planes;
+	int ps_s, ps_oc, ps_w; /* pixel shuffle (struct s3k_gemm), ps_s 0 = none */
 	int tstrip;   /* tile order (tile_of): 0, or N strips of this many tiles */
 	int xwalk;    /* each slice's tiles on one XCD: gemm_dlk 1; gemm_dlt the
 		       * slice count of its grouped 1-D grid; 0 off */
@@ -562,7 +563,7 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 	if (FIXED && (flags & S3K_EPI_BIAS)) {
 		const int cw = (lane % (WTN / W)) * W;
 		if (n0 + cw < p.N)
-			epi_bias<W>(p, n0 + cw, ein.b);
+			epi_bias<W>(p, p.ps_s ? (n0 + cw) % p.ps_oc : n0 + cw, ein.b);
 	}
 	/* staged values of unit s: row s / (WTN / W), columns cw.. cw + W - 1 */
 	auto staged = [&](int s, float (&x)[W]) {
@@ -598,6 +599,35 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 	auto fast_strips = [&](auto eb_t, auto eg_t) {
 		constexpr bool EB = decltype(eb_t)::value, EG = decltype(eg_t)::value;
 		constexpr int IT = UNITS / 64;
+		/* pixel shuffle: the lane's tap and channel are the same for the
+		 * whole tile, its pixel (py, px) steps by RPI rows per store */
+		constexpr bool PS_CK = FIXED && (CK == S3K_F32 || CK == S3K_C_PLANES);
+		constexpr int RPI = FIXED ? 64 / (WTN / W) : 1;
+		int py = 0, px = 0, ptap = 0, pcol = 0;
+		const int plane = PS_CK && p.ps_s ? p.ps_oc : p.N;
+		if constexpr (PS_CK) {
+			if (p.ps_s) {
+				const int m1 = m0 + lane / (WTN / W), n = n0 + (lane % (WTN / W)) * W;
+				const int t = n / p.ps_oc, kh = t / p.ps_s;
+				pcol = n - t * p.ps_oc;
+				ptap = kh * p.ps_w * p.ps_s + (t - kh * p.ps_s);
+				py = m1 / p.ps_w;
+				px = m1 - py * p.ps_w;
+			}
+		}
+		/* element offset of this store's first value */
+		auto place = [&](int m, int n) -> long long {
+			if constexpr (PS_CK) {
+				if (p.ps_s) {
+					const long long r = (long long)py * p.ps_s * (p.ps_w * p.ps_s) +
+							    px * p.ps_s + ptap;
+					for (px += RPI; px >= p.ps_w; px -= p.ps_w)
+						++py;
+					return r * p.ldc + pcol;
+				}
+			}
+			return (long long)m * p.ldc + n;
+		};
 #pragma unroll
 		for (int i = 0; i < FM; ++i) {
 			stage(acc[i]);
@@ -636,10 +666,11 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 							f16_row_tag(p, m, mx);
 					}
 				}
+				const long long o = place(m, n);
 				if constexpr (OPERAND_CK) {
 					/* plain stores: the next GEMM reads them at once */
 					if (m < p.M) {
-						uint16_t *c = (uint16_t *)cb + (long long)m * p.ldc + n;
+						uint16_t *c = (uint16_t *)cb + o;
 						uint32_t hi[4], lo[4];
 #pragma unroll
 						for (int e = 0; e < 4; ++e) {
@@ -651,8 +682,8 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 						}
 						*(s3k_u32x4 *)c = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
 						if constexpr (CK == S3K_C_PLANES) {
-							*(s3k_u32x4 *)(c + p.N) = (s3k_u32x4){lo[0], lo[1], lo[2], lo[3]};
-							*(s3k_u32x4 *)(c + 2LL * p.N) = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
+							*(s3k_u32x4 *)(c + plane) = (s3k_u32x4){lo[0], lo[1], lo[2], lo[3]};
+							*(s3k_u32x4 *)(c + 2LL * plane) = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
 						}
 					}
 				} else if (m < p.M) {
@@ -666,7 +697,6 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 					 * and residual sums are read by the next kernel
 					 * at once, and streaming stores there made the
 					 * ViT block 3 % slower. */
-					const long long o = (long long)m * p.ldc + n;
 					if constexpr (CK == S3K_F32) {
 						__builtin_nontemporal_store((s3k_f32x4){v[it][0], v[it][1], v[it][2], v[it][3]},
 									    (s3k_f32x4 *)((float *)cb + o));

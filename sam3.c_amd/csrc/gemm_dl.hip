@@ -986,10 +986,12 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 	 * tile */
 	if ((g->flags & S3K_EPI_QKV) && (cfg < 20 || cfg == 25))
 		cfg = 26;
-	if ((s3h_settings()->dl_cfg < 0 || cfg == 30) && dlk_ok(g))
+	if (g->ps_s && cfg == 25) /* 96-column wave tiles: not the unrolled stores */
+		cfg = 24;
+	if ((s3h_settings()->dl_cfg < 0 || cfg == 30) && !g->ps_s && dlk_ok(g))
 		return g->a_kind == S3K_BF16 ? launch_dlk<FAM_BF16, 3>(g, p, st)
 					     : launch_dlk<FAM_F16, 3>(g, p, st);
-	if (cfg == 31 && dlk_ok(g))
+	if (cfg == 31 && !g->ps_s && dlk_ok(g))
 		return g->a_kind == S3K_BF16 ? launch_dlk<FAM_BF16, 2>(g, p, st)
 					     : launch_dlk<FAM_F16, 2>(g, p, st);
 	if (cfg == 30 || cfg == 31)

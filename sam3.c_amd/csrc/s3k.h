@@ -129,6 +129,14 @@ struct s3k_gemm {
 	 * >= 4, qkv_S >= 32, N = E, 2E or 3E, M a multiple of qkv_S. When
 	 * bit y of qkv_planes is set (qkv_D = 64, not the skinny kernel),
 	 * each row of operand y is stored as planes (s3k_attn_heads, kvp). */
+	/* pixel shuffle (ps_s > 0): a transposed convolution with stride =
+	 * kernel = ps_s, N = ps_s^2 taps x ps_oc channels, row m the pixel
+	 * (m / ps_w, m % ps_w): column n, tap (kh, kw) = divmod(n / ps_oc,
+	 * ps_s), goes to column n % ps_oc of output row ((m / ps_w) * ps_s +
+	 * kh) * (ps_w * ps_s) + (m % ps_w) * ps_s + kw, with bias[ps_oc];
+	 * ldc and the planes' distance are those of ps_oc columns. ps_oc a
+	 * multiple of 64, direct-to-LDS GEMM, f32 or S3K_C_PLANES output */
+	int          ps_s, ps_oc, ps_w;
 	float       *qkv_out[3];
 	const float *qkv_cos, *qkv_sin;
 	int          qkv_S, qkv_H, qkv_D, qkv_rope, qkv_planes;
@@ -335,6 +343,7 @@ struct s3k_conv {
 	void       *y;
 	const void *bias;
 	int kind, flags;
+	int out_planes; /* f32 implicit GEMM, OC % 8 == 0: y as S3K_C_PLANES rows */
 	int N, H, W, C, OC, KH, KW, stride, pad_h, pad_w, groups, OH, OW;
 };
 int s3k_conv_implicit(const struct s3k_conv *c, const void *xa, const void *wb, int pixel_pitch,

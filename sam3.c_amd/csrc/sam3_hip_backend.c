@@ -1544,6 +1544,47 @@ static enum sam3_error run_layernorm_as(struct sam3_hip_backend *hb, const struc
 /* CONV2D or CONV_TRANSPOSE2D at node i, plus a following BIAS_ADD ([OC],
  * used only there) and GELU folded into the GEMM epilogue when the conv
  * runs as a GEMM. */
+/* Whether the f32 result `out` of the (transposed) convolution folded up to
+ * node j may be written as bf16 planes: one node reads it (under any
+ * header), a (transposed) convolution taking it as its input planes, whose
+ * weight no node of the graph writes. */
+static int conv_planes_reader(struct sam3_hip_backend *hb, const struct sam3_graph *g, int j,
+			      const struct sam3_tensor *out, struct use_map *uses)
+{
+	static const char al[16] __attribute__((aligned(16)));
+	const struct s3h_settings *set = s3h_settings();
+	if (!set->gemm_operand || set->readback_all || out->dtype != SAM3_DTYPE_F32 ||
+	    uses_of(uses, out) != 1)
+		return 0;
+	const int k = next_reader(g, j, out);
+	const struct sam3_node *n = k >= 0 ? &g->nodes[k] : NULL;
+	if (!n || (n->op != SAM3_OP_CONV2D && n->op != SAM3_OP_CONV_TRANSPOSE2D) || n->inputs[0] != out ||
+	    n->n_inputs < 2 || !n->inputs[1] || !n->output || same_data(n->inputs[1], out))
+		return 0;
+	for (int m = 0; m < g->n_nodes; m++) {
+		const struct sam3_node *o = &g->nodes[m];
+		if (same_data(o->output, n->inputs[1]) ||
+		    (m >= j && m < k && same_data(o->output, out)))
+			return 0;
+		for (int r = 0; m != k && m >= j && r < o->n_inputs && r < SAM3_NODE_MAX_INPUTS; r++)
+			if (same_data(o->inputs[r], out))
+				return 0;
+	}
+	struct sam3_tensor tx = *out, tw = *n->inputs[1], ty = *n->output;
+	struct sam3_node dn = *n;
+	tx.data = ty.data = (void *)al;
+	if (dev_in(hb, n->inputs[1], &tw.data) != SAM3_OK)
+		return 0;
+	dn.inputs[0] = &tx;
+	dn.inputs[1] = &tw;
+	dn.output = &ty;
+	/* the reader's own output address decides its path as well, and a
+	 * caller may have put it anywhere on the device */
+	if ((uintptr_t)n->output->data & 15u)
+		return 0;
+	return n->op == SAM3_OP_CONV2D ? s3h_conv2d_planes_in(&dn) : s3h_conv_transpose2d_planes(&dn);
+}
+
 static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_graph *g, int i,
 				struct use_map *uses, int *used)
 {
@@ -1551,6 +1592,8 @@ static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_g
 	const struct sam3_node *n = &g->nodes[i];
 	struct sam3_tensor tx = *n->inputs[0], tw = *n->inputs[1], ty = *n->output;
 	struct sam3_node dn = *n;
+	const struct s3h_res *xe = res_find(hb, n->inputs[0]->data);
+	const int x_planes = xe && xe->fmt == S3H_A_PLANES;
 	enum sam3_error err = dev_in(hb, n->inputs[0], &tx.data);
 	if (err == SAM3_OK)
 		err = dev_in(hb, n->inputs[1], &tw.data);
@@ -1585,13 +1628,19 @@ static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_g
 	void *dbias = NULL;
 	if (bias)
 		err = dev_in(hb, bias, &dbias);
-	if (err == SAM3_OK)
-		err = dev_out(hb, out, &ty.data);
 	if (err != SAM3_OK)
 		return err;
-	err = transposed ? s3h_conv_transpose2d(&dn, dbias, flags, path, hb->stream)
-			 : s3h_conv2d(&dn, dbias, flags, path, hb->stream);
+	/* a result only the next convolution reads: written as its planes */
+	const int out_planes = (transposed ? s3h_conv_transpose2d_planes(&dn) : s3h_conv2d_planes_out(&dn)) &&
+			       conv_planes_reader(hb, g, j, out, uses);
+	err = out_planes ? dev_out_fmt(hb, out, (size_t)ny * 6, S3H_A_PLANES, &ty.data, NULL)
+			 : dev_out(hb, out, &ty.data);
+	if (err != SAM3_OK)
+		return err;
+	err = transposed ? s3h_conv_transpose2d(&dn, dbias, flags, path, x_planes, out_planes, hb->stream)
+			 : s3h_conv2d(&dn, dbias, flags, path, x_planes, out_planes, hb->stream);
 	if (err == SAM3_OK) {
+		hb->stats.operand_writes += out_planes;
 		hb->stats.gpu_nodes++;
 		hb->stats.fused_nodes += j - i - 1;
 		*used = j - i;

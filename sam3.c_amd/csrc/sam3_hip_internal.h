@@ -68,8 +68,13 @@ int s3h_sdpa_node_ok(const struct sam3_node *node);
 enum { S3H_CONV_IMPLICIT = 1, S3H_CONV_IM2COL = 2, S3H_CONV_DIRECT = 3 };
 int s3h_conv2d_ok(const struct sam3_node *node);
 int s3h_conv2d_path(const struct sam3_node *node);
+/* x_planes: the input's data are bf16 planes (S3H_A_PLANES rows of C);
+ * out_planes: the output is written so (rows of OC). Only where
+ * s3h_conv2d_planes_in / _planes_out say so. */
 enum sam3_error s3h_conv2d(const struct sam3_node *node, const void *bias, int flags, int path,
-			   void *stream);
+			   int x_planes, int out_planes, void *stream);
+int s3h_conv2d_planes_in(const struct sam3_node *node);
+int s3h_conv2d_planes_out(const struct sam3_node *node);
 /* CONV_TRANSPOSE2D and MAXPOOL2D (NHWC, F32). s3h_conv_transpose2d runs
  * path 0 (the best), S3H_CONVT_GEMM (stride = KH = KW, pad 0: one GEMM and
  * a pixel-shuffle permute; bias/flags fold a BIAS_ADD and GELU) or
@@ -78,7 +83,10 @@ enum { S3H_CONVT_GEMM = 1, S3H_CONVT_DIRECT = 3 };
 int s3h_conv_transpose2d_ok(const struct sam3_node *node);
 int s3h_conv_transpose2d_path(const struct sam3_node *node);
 enum sam3_error s3h_conv_transpose2d(const struct sam3_node *node, const void *bias, int flags,
-				     int path, void *stream);
+				     int path, int x_planes, int out_planes, void *stream);
+/* Whether it takes and writes planes (one condition: the split GEMM with
+ * the pixel shuffle in its epilogue runs it). */
+int s3h_conv_transpose2d_planes(const struct sam3_node *node);
 int s3h_maxpool2d_ok(const struct sam3_node *node);
 enum sam3_error s3h_maxpool2d(const struct sam3_node *node, void *stream);
 int s3h_bias_add_ok(const struct sam3_node *node);

@@ -2192,7 +2192,7 @@ static enum sam3_error free_scratch(void *p, void *stream, enum sam3_error err)
 
 /* Conv on device pointers; bias ([OC], the conv's dtype) and GELU are
  * applied in the GEMM epilogue (paths 1 and 2 only). */
-static enum sam3_error conv_run(struct s3k_conv *c, int path, void *stream)
+static enum sam3_error conv_run(struct s3k_conv *c, int path, int x_planes, void *stream)
 {
 	const int f32 = c->kind == SAM3_DTYPE_F32;
 	const int K = c->KH * c->KW * c->C;
@@ -2210,15 +2210,17 @@ static enum sam3_error conv_run(struct s3k_conv *c, int path, void *stream)
 		const long long pix = (long long)c->N * c->H * c->W;
 		void *xp = NULL, *wp = NULL;
 		int own_w = 0;
-		err = s3h_scratch_alloc(&xp, (size_t)pix * 3 * c->C * 2, stream);
+		if (!x_planes)
+			err = s3h_scratch_alloc(&xp, (size_t)pix * 3 * c->C * 2, stream);
 		if (err == SAM3_OK)
 			err = prep_weight(c->w, (size_t)c->OC * K * 4, S3H_PREP_SPLIT_W, c->OC, K, K,
 					  (size_t)c->OC * 3 * K * 2, S3K_F32, prep_split_w, stream, &wp, &own_w);
-		if (err == SAM3_OK)
+		if (err == SAM3_OK && !x_planes)
 			err = s3h_hip(s3k_split3_bf16((const float *)c->x, xp, (int)pix, c->C, c->C, 0, stream),
 				      "conv2d split x");
 		if (err == SAM3_OK)
-			err = s3h_hip(s3k_conv_implicit(c, xp, wp, 3 * c->C, stream), "conv2d implicit");
+			err = s3h_hip(s3k_conv_implicit(c, x_planes ? c->x : xp, wp, 3 * c->C, stream),
+				      "conv2d implicit");
 		return free_scratch(xp, stream, free_scratch(own_w ? wp : NULL, stream, err));
 	}
 	/* path 2: column matrix [M, Kp] (or planes [M, 3Kp]) and the NT GEMM */
@@ -2266,8 +2268,25 @@ int s3h_conv2d_path(const struct sam3_node *node)
 	return conv_shape(node, &c, 1) == SAM3_OK ? conv_path_of(&c) : 0;
 }
 
+static int conv_planes_fit(const struct sam3_node *node)
+{
+	struct s3k_conv c;
+	return conv_shape(node, &c, 1) == SAM3_OK && c.kind == SAM3_DTYPE_F32 &&
+	       conv_path_of(&c) == S3H_CONV_IMPLICIT;
+}
+
+int s3h_conv2d_planes_in(const struct sam3_node *node)
+{
+	return conv_planes_fit(node);
+}
+
+int s3h_conv2d_planes_out(const struct sam3_node *node)
+{
+	return conv_planes_fit(node) && node->inputs[1]->dims[0] % 8 == 0;
+}
+
 enum sam3_error s3h_conv2d(const struct sam3_node *node, const void *bias, int flags, int path,
-			   void *stream)
+			   int x_planes, int out_planes, void *stream)
 {
 	struct s3k_conv c;
 	enum sam3_error err = conv_shape(node, &c, 0);
@@ -2287,17 +2306,23 @@ enum sam3_error s3h_conv2d(const struct sam3_node *node, const void *bias, int f
 		s3h_error("conv2d: NULL bias");
 		return SAM3_EINVAL;
 	}
-	return conv_run(&c, path, stream);
+	if ((x_planes || out_planes) &&
+	    (path != S3H_CONV_IMPLICIT || c.kind != SAM3_DTYPE_F32 || (out_planes && c.OC % 8))) {
+		s3h_error("conv2d: planes on path %d", path);
+		return SAM3_EINVAL;
+	}
+	c.out_planes = out_planes;
+	return conv_run(&c, path, x_planes, stream);
 }
 
 enum sam3_error sam3_hip_kernel_conv2d(const struct sam3_node *node, void *stream)
 {
-	return s3h_conv2d(node, NULL, 0, 0, stream);
+	return s3h_conv2d(node, NULL, 0, 0, 0, 0, stream);
 }
 
 enum sam3_error sam3_hip_conv2d_on_path(int path, const struct sam3_node *node, void *stream)
 {
-	return s3h_conv2d(node, NULL, 0, path, stream);
+	return s3h_conv2d(node, NULL, 0, path, 0, 0, stream);
 }
 
 int sam3_hip_conv2d_path(const struct sam3_node *node)
@@ -2434,8 +2459,32 @@ static int prep_convt_w(const void *w, void *out, int rows, int k, int k_out, in
 	return s3k_permute(4, w, out, 3, dims, axes, stream);
 }
 
+/* The GEMM of convt_gemm_ok's c as the split f32 GEMM storing y itself
+ * (struct s3k_gemm, ps_*): its epilogue writes whole 64-channel runs. */
+static int convt_shuffle_gemm(const struct convt_shape *c, const void *wt, const void *bias, int flags,
+			      struct s3k_gemm *g)
+{
+	const int M = c->N * c->H * c->W, NN = c->KH * c->KW * c->OC;
+	fill_gemm(g, SAM3_DTYPE_F32, c->x, SAM3_DTYPE_F32, wt, SAM3_DTYPE_F32, c->y, M, NN, c->C, bias,
+		  (flags & (S3K_EPI_BIAS | S3K_EPI_GELU)) | SAM3_HIP_B_NT);
+	g->ps_s = c->stride;
+	g->ps_oc = c->OC;
+	g->ps_w = c->W;
+	return c->OC % 64 == 0 && f32_split_wanted(g);
+}
+
+int s3h_conv_transpose2d_planes(const struct sam3_node *node)
+{
+	static const char al[16] __attribute__((aligned(16)));
+	struct convt_shape c;
+	struct s3k_gemm g;
+	return convt_shape(node, &c, 1) == SAM3_OK && convt_path_of(&c) == S3H_CONVT_GEMM &&
+	       convt_shuffle_gemm(&c, al, NULL, 0, &g) &&
+	       (long long)c.N * c.H * c.W * c.KH * c.KW * c.OC * 6 <= 0x7FFFFFF0LL;
+}
+
 enum sam3_error s3h_conv_transpose2d(const struct sam3_node *node, const void *bias, int flags,
-				     int path, void *stream)
+				     int path, int x_planes, int out_planes, void *stream)
 {
 	struct convt_shape c;
 	enum sam3_error err = convt_shape(node, &c, 0);
@@ -2461,13 +2510,29 @@ enum sam3_error s3h_conv_transpose2d(const struct sam3_node *node, const void *b
 		return SAM3_EINVAL;
 	}
 	/* Each input pixel times W' [taps*OC, C] gives its taps' output
-	 * pixels: tmp [N*H*W, taps*OC], then [N*H, W, KH, KW*OC] ->
-	 * [N*H, KH, W, KW*OC] is y. */
+	 * pixels: stored in place by the GEMM's epilogue, or (channels not a
+	 * multiple of 64, small problems) tmp [N*H*W, taps*OC], then
+	 * [N*H, W, KH, KW*OC] -> [N*H, KH, W, KW*OC] is y. */
 	const int T = c.KH * c.KW, M = c.N * c.H * c.W, NN = T * c.OC;
 	void *wt = NULL, *tmp = NULL, *b4 = NULL;
 	int own_w = 0;
 	err = prep_weight(c.w, (size_t)c.OC * T * c.C * 4, S3H_PREP_CONVT_W, c.OC, c.C, T,
 			  (size_t)NN * c.C * 4, S3K_F32, prep_convt_w, stream, &wt, &own_w);
+	struct s3k_gemm sg;
+	if (err == SAM3_OK && convt_shuffle_gemm(&c, wt, bias, flags, &sg)) {
+		if (out_planes) {
+			sg.c_kind = S3K_C_PLANES;
+			sg.ldc = 3 * c.OC;
+		} else {
+			sg.ldc = c.OC;
+		}
+		err = f32_split_gemm(&sg, x_planes ? c.x : NULL, stream);
+		return free_scratch(own_w ? wt : NULL, stream, err);
+	}
+	if (err == SAM3_OK && (x_planes || out_planes)) {
+		s3h_error("conv_transpose2d: planes without the shuffling GEMM");
+		err = SAM3_EINVAL;
+	}
 	if (err == SAM3_OK)
 		err = s3h_scratch_alloc(&tmp, (size_t)M * NN * 4, stream);
 	if (err == SAM3_OK && (flags & S3K_EPI_BIAS)) {
@@ -2490,13 +2555,13 @@ enum sam3_error s3h_conv_transpose2d(const struct sam3_node *node, const void *b
 
 enum sam3_error sam3_hip_kernel_conv_transpose2d(const struct sam3_node *node, void *stream)
 {
-	return s3h_conv_transpose2d(node, NULL, 0, 0, stream);
+	return s3h_conv_transpose2d(node, NULL, 0, 0, 0, 0, stream);
 }
 
 enum sam3_error sam3_hip_conv_transpose2d_on_path(int path, const struct sam3_node *node,
 						  void *stream)
 {
-	return s3h_conv_transpose2d(node, NULL, 0, path, stream);
+	return s3h_conv_transpose2d(node, NULL, 0, path, 0, 0, stream);
 }
 
 int sam3_hip_conv_transpose2d_path(const struct sam3_node *node)
@@ -2775,7 +2840,7 @@ enum sam3_error sam3_hip_dispatch_node(const struct sam3_node *node, void *strea
 		break;
 	case SAM3_OP_CONV2D:
 		if (is_float_dtype(dtype))
-			return s3h_conv2d(node, NULL, 0, 0, stream);
+			return s3h_conv2d(node, NULL, 0, 0, 0, 0, stream);
 		break;
 	case SAM3_OP_BIAS_ADD:
 		if (is_float_dtype(dtype))
@@ -2783,7 +2848,7 @@ enum sam3_error sam3_hip_dispatch_node(const struct sam3_node *node, void *strea
 		break;
 	case SAM3_OP_CONV_TRANSPOSE2D:
 		if (dtype == SAM3_DTYPE_F32)
-			return s3h_conv_transpose2d(node, NULL, 0, 0, stream);
+			return s3h_conv_transpose2d(node, NULL, 0, 0, 0, 0, stream);
 		break;
 	case SAM3_OP_MAXPOOL2D:
 		if (dtype == SAM3_DTYPE_F32)

@@ -292,3 +292,73 @@ def test_neck_stage_4x_in_graph():
     r = O.bias_add(O.conv2d(r, w3, 1, 0).reshape(-1, 64), b3, "f32").reshape(1, 48, 48, 64)
     r = O.bias_add(O.conv2d(r, w4, 1, 1).reshape(-1, 64), b4, "f32").reshape(1, 48, 48, 64)
     assert_f32_close(got, r, what="neck 4x stage")
+
+
+@pytest.mark.parametrize("cfg", [2, 6, 7])
+@pytest.mark.parametrize("name", ["c128_1x1", "c64_s2_tail", "c192_oc20"])
+def test_conv2d_deep_ring_tiles(env, name, cfg):
+    """The 64x64 implicit-GEMM tiles with two (cfg 2), four (6) and three
+    (7) LDS stages on fewer k-steps than stages and more, ragged rows and
+    columns: the same bits, near the oracle."""
+    xs, ws, st, ph, pw, gr, _ = CASES[name]
+    for kind in ("f32", "bf16"):
+        x, w = cast(synth.randn(310, xs), kind), cast(synth.randn(311, ws, 0.1), kind)
+        env.set("SAM3_HIP_CONV_CFG", cfg)
+        got = gpu_conv(x, w, st, ph, pw, gr, kind, IMPLICIT)
+        env.set("SAM3_HIP_CONV_CFG", 4)
+        assert np.array_equal(got, gpu_conv(x, w, st, ph, pw, gr, kind, IMPLICIT))
+        check(got, oracle().conv2d(x, w, st, ph, pw, gr, kind=kind), kind, False, f"{name} {cfg}")
+
+
+@pytest.mark.parametrize("h,w,dim,d", [(13, 11, 512, 64), (13, 20, 768, 128), (5, 33, 512, 72)])
+def test_conv_chain_writes_planes(env, h, w, dim, d):
+    """ConvT (GELU) -> ConvT -> 1x1 -> 3x3 with biases in one graph: each
+    result is written as the next node's planes, the transposed convolutions
+    store their taps in place. Odd widths, ragged M, channel counts of one
+    and several 64-column runs (72: the 3x3 takes the column matrix, so the
+    1x1 writes f32 rows of 72);
+    the bits of separate split and shuffle passes
+    (SAM3_HIP_GEMM_OPERAND=0), and near the oracle."""
+    from sam3_amd import graph
+    from test_gpu_blockops import C as CT
+    O, F = oracle(), abi.F32
+    x = synth.randn(320, (1, h, w, dim))
+    plan = [("T", dim // 2, 2, True), ("T", dim // 4, 2, False), ("C", d, 1, False), ("C", d, 3, False)]
+
+    def run(mode):
+        env.set("SAM3_HIP_GEMM_OPERAND", mode)
+        G = graph.Graph()
+        t, ref, c, hh, ww = G.tensor(F, x.shape, x), x, dim, h, w
+        for i, (op, oc, k, gelu) in enumerate(plan):
+            wt, b = synth.randn(321 + 2 * i, (oc, k, k, c), 0.05), synth.randn(322 + 2 * i, (oc,), 0.1)
+            tw, tb = G.tensor(F, wt.shape, wt), G.tensor(F, b.shape, b)
+            if op == "T":
+                hh, ww = 2 * hh, 2 * ww
+                t = G.node(abi.OP_CONV_TRANSPOSE2D, [t, tw], G.tensor(F, (1, hh, ww, oc)), (2, 0, 0, 0))
+                ref = O.conv_transpose2d(ref, wt, 2, 0)
+            else:
+                t = G.node(abi.OP_CONV2D, [t, tw], G.tensor(F, (1, hh, ww, oc)), (1, k // 2, 1, 0))
+                ref = O.conv2d(ref, wt, 1, k // 2, None, 1, kind="f32")
+            t = G.node(abi.OP_BIAS_ADD, [t, tb], G.tensor(F, (1, hh, ww, oc)))
+            ref = ref + b
+            if gelu:
+                t = G.node(abi.OP_GELU, [t], G.tensor(F, (1, hh, ww, oc)))
+                u = 0.7978845608 * (ref + 0.044715 * ref.astype(np.float64) ** 3)
+                ref = (0.5 * ref * (1 + np.tanh(u))).astype(np.float32)
+            c = oc
+        be = hip.Backend(0)
+        try:
+            assert be.graph_eval(G.g) == abi.OK
+            st = be.stats()
+            got = np.ctypeslib.as_array(CT.cast(t.data, CT.POINTER(CT.c_float)),
+                                        shape=(1, hh, ww, c)).copy()
+        finally:
+            be.close()
+        return got, ref, st
+
+    a, ref, st = run("1")
+    b, _, st0 = run("0")
+    assert st.host_nodes == 0 and st0.operand_writes == 0
+    assert st.operand_writes == (3 if d % 64 == 0 else 2)
+    assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
+    assert_f32_close(a, ref, what="conv chain")
