@@ -49,8 +49,8 @@ struct AttnArgs {
 	int mask_vec;           /* mask rows 16-byte aligned: float4 loads */
 	int oh;                 /* > 0: output head-merged (at_out_row)      */
 	int ofmt;               /* merged f32 rows written as a GEMM operand:
-				 * 0 f32, 1 bf16 planes [hi|lo|hi] (row pitch
-				 * 3*oh*D), 2 f16 with the range flag        */
+				 * 0 f32, 1 bf16 planes [hi|lo] (row pitch
+				 * 2*oh*D), 2 f16 with the range flag        */
 	unsigned *ovf;          /* ofmt 2: range flag (or NULL) and its tag  */
 	unsigned ovf_tag;
 };
@@ -204,13 +204,12 @@ __device__ __forceinline__ void at_store(const AttnArgs &p, const s3k_f32x16 (&o
 						/* the merged row r = orow / K as bf16 planes,
 						 * the split of split3 / the permute kernel */
 						const long long K = (long long)p.oh * AT_D, r = orow / K;
-						uint16_t *dp = (uint16_t *)p.out + r * 3 * K + (orow - r * K) + d0;
+						uint16_t *dp = (uint16_t *)p.out + r * 2 * K + (orow - r * K) + d0;
 						uint32_t hi[2], lo[2];
 						split_bf16x2(x0, x1, hi[0], lo[0]);
 						split_bf16x2(x2, x3, hi[1], lo[1]);
 						*(uint2 *)dp = make_uint2(hi[0], hi[1]);
 						*(uint2 *)(dp + K) = make_uint2(lo[0], lo[1]);
-						*(uint2 *)(dp + 2 * K) = make_uint2(hi[0], hi[1]);
 					} else if (p.ofmt == 2) {
 						/* f16, flagged as the permute kernel flags it: a
 						 * value past 2^15, or four nonzero values all
@@ -1326,15 +1325,14 @@ __global__ void __launch_bounds__(256) attn_small(AttnGArgs p)
 		if (p.ofmt == 0) {
 			((float *)p.out)[orow + lane] = x;
 		} else if (p.ofmt == 1) {
-			/* bf16 planes [hi|lo|hi] of the merged row, as attn_fwd */
+			/* bf16 planes [hi|lo] of the merged row, as attn_fwd */
 			if (!(lane & 1)) {
 				const long long K = (long long)p.oh * AT_D, r = orow / K;
-				uint16_t *dp = (uint16_t *)p.out + r * 3 * K + (orow - r * K) + lane;
+				uint16_t *dp = (uint16_t *)p.out + r * 2 * K + (orow - r * K) + lane;
 				uint32_t hi, lo;
 				split_bf16x2(x, x1, hi, lo);
 				*(uint32_t *)dp = hi;
 				*(uint32_t *)(dp + K) = lo;
-				*(uint32_t *)(dp + 2 * K) = hi;
 			}
 		} else {
 			/* f16, flagged per four values as attn_fwd flags them */

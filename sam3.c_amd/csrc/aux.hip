@@ -615,10 +615,11 @@ extern "C" int s3k_q8_dequantize(const void *src, void *dst, int n, void *stream
 	return (int)hipGetLastError();
 }
 
-/* f32 rows [rows, K] (row pitch ld elements) -> bf16 rows [rows, 3K] of
- * hi = bf16(x) and lo = bf16(x - hi) in the order [hi, lo, hi] (order 0)
- * or [hi, hi, lo] (order 1): a bf16 GEMM of one against the other over
- * 3K sums hi*hi + lo*hi + hi*lo. One thread per 8 values of a row. */
+/* f32 rows [rows, K] (row pitch ld elements) -> bf16 rows of hi = bf16(x)
+ * and lo = bf16(x - hi): [hi, lo] when K is a multiple of 64 (s3k_planes),
+ * else in the order [hi, lo, hi] (order 0) or [hi, hi, lo] (order 1): a
+ * bf16 GEMM of one against the other over 3K sums hi*hi + lo*hi + hi*lo.
+ * One thread per 8 values of a row. */
 __global__ void __launch_bounds__(256) split3_bf16_k(const float *src, uint16_t *dst, int rows,
 						     int K, long long ld, int order)
 {
@@ -635,9 +636,11 @@ __global__ void __launch_bounds__(256) split3_bf16_k(const float *src, uint16_t 
 	split_bf16x2(a.z, a.w, H.y, L.y);
 	split_bf16x2(b.x, b.y, H.z, L.z);
 	split_bf16x2(b.z, b.w, H.w, L.w);
-	uint16_t *d = dst + r * 3LL * K + k0;
+	uint16_t *d = dst + r * (K & 63 ? 3LL : 2LL) * K + k0;
 	*(uint4 *)d = H;
-	if (order == 0) {
+	if ((K & 63) == 0) {
+		*(uint4 *)(d + K) = L;
+	} else if (order == 0) {
 		*(uint4 *)(d + K) = L;
 		*(uint4 *)(d + 2LL * K) = H;
 	} else {

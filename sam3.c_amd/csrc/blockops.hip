@@ -142,10 +142,11 @@ __global__ void __launch_bounds__(256) layernorm_k(const void *x, const void *ga
 		} else if constexpr (OUTF == S3K_LN_PLANES) {
 			uint32_t hi, lo;
 			split_bf16x2(val, 0.0f, hi, lo);
-			uint16_t *d = (uint16_t *)out + orow * 3LL * cols + j;
+			uint16_t *d = (uint16_t *)out + orow * (cols & 63 ? 3LL : 2LL) * cols + j;
 			d[0] = (uint16_t)hi;
 			d[cols] = (uint16_t)lo;
-			d[2LL * cols] = (uint16_t)hi;
+			if (cols & 63) /* s3k_planes */
+				d[2LL * cols] = (uint16_t)hi;
 		} else {
 			((uint16_t *)out)[obase + j] = (uint16_t)f32_to_f16(val);
 		}
@@ -259,10 +260,10 @@ __global__ void __launch_bounds__(256) layernorm_v(const void *x, const void *ga
 			uint32_t hi[2], lo[2];
 			split_bf16x2(v[i][0], v[i][1], hi[0], lo[0]);
 			split_bf16x2(v[i][2], v[i][3], hi[1], lo[1]);
-			uint16_t *d = (uint16_t *)out + orow * 3LL * cols + j0;
+			/* rows of 256 values and up here: two planes (s3k_planes) */
+			uint16_t *d = (uint16_t *)out + orow * 2LL * cols + j0;
 			*(uint2 *)d = make_uint2(hi[0], hi[1]);
 			*(uint2 *)(d + cols) = make_uint2(lo[0], lo[1]);
-			*(uint2 *)(d + 2LL * cols) = make_uint2(hi[0], hi[1]);
 		} else {
 			*(uint2 *)((uint16_t *)out + obase + j0) =
 				make_uint2(pack_f16x2(v[i][0], v[i][1]), pack_f16x2(v[i][2], v[i][3]));
@@ -394,10 +395,11 @@ __global__ void __launch_bounds__(256) permute_op_k(PermArgs a, unsigned K)
 			uint32_t hi[2], lo[2];
 			split_bf16x2(v.x, v.y, hi[0], lo[0]);
 			split_bf16x2(v.z, v.w, hi[1], lo[1]);
-			uint16_t *d = (uint16_t *)a.dst + (e / K) * 3LL * K + e % K;
+			uint16_t *d = (uint16_t *)a.dst + (e / K) * (K & 63 ? 3LL : 2LL) * K + e % K;
 			*(uint2 *)d = make_uint2(hi[0], hi[1]);
 			*(uint2 *)(d + K) = make_uint2(lo[0], lo[1]);
-			*(uint2 *)(d + 2LL * K) = make_uint2(hi[0], hi[1]);
+			if (K & 63) /* s3k_planes */
+				*(uint2 *)(d + 2LL * K) = make_uint2(hi[0], hi[1]);
 		} else {
 			/* a value past 2^15, or four nonzero values all below 2^-10:
 			 * the f16 copy would not hold them to f16 precision */

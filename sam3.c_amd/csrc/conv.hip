@@ -17,9 +17,9 @@
  *     the padding get an out-of-range buffer offset and load zeros. The
  *     column matrix is never written.
  *     f32 tensors run on bf16 planes, as the split f32 GEMM does: x is
- *     split once into [hi|lo|hi] per pixel (pixel pitch 3C) and W into
- *     [hi|hi|lo] per row, and the virtual k' = 3K walks the three planes,
- *     so the accumulator sums hi*hi + lo*hi + hi*lo.
+ *     split once into [hi|lo] per pixel (pixel pitch 2C) and W into
+ *     [hi|lo] per row, and the virtual k' = 3K walks hi, lo, hi against
+ *     hi, hi, lo, so the accumulator sums hi*hi + lo*hi + hi*lo.
  *   conv_im2col_k + GEMM (groups 1, other C, e.g. the patch embedding's
  *     C = 3): the column matrix in 16-bit, or in the f32 planes, with K
  *     padded to a multiple of 8 for gemm_dl; conv_wprep_k pads (and
@@ -36,7 +36,7 @@ namespace s3k {
 struct ConvArgs {
 	GemmArgs g;    /* a = x or its planes, b = W [OC, K'], c = y; M = N*OH*OW, N = OC, K = K' */
 	int H, W, C, KH, KW, stride, ph, pw, OH, OW;
-	int PP;        /* pixel pitch of the A source in elements (C, or 3C for f32 planes) */
+	int PP;        /* pixel pitch of the A source in elements (C, or 2C for f32 planes) */
 };
 
 template <int CPR>
@@ -110,7 +110,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) conv_dl(ConvArgs q)
 	auto issue = [&](int kt) {
 		const int k0 = kt * BK;
 		const unsigned st = lds0 + (unsigned)((kt % STAGES) * SB) + (unsigned)wave * 1024u;
-		const int toff = ((w_kh * q.W + w_kw) * q.PP + w_seg * q.C + w_ic) * 2;
+		/* plane of segment 0, 1, 2: hi, lo, hi */
+		const int toff = ((w_kh * q.W + w_kw) * q.PP + (w_seg == 1 ? q.C : 0) + w_ic) * 2;
 #pragma unroll
 		for (int j = 0; j < A_PER; ++j) {
 			const int ih = a_ih[j] + w_kh, iw = a_iw[j] + w_kw;
@@ -119,7 +120,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) conv_dl(ConvArgs q)
 		}
 #pragma unroll
 		for (int j = 0; j < B_PER; ++j)
-			dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], 2u * k0);
+			dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b(p, k0));
 		w_ic += BK;
 		if (w_ic == q.C) {
 			w_ic = 0;
@@ -374,7 +375,8 @@ extern "C" int s3k_conv_implicit(const struct s3k_conv *c, const void *xa, const
 	const long long M = (long long)c->N * c->OH * c->OW;
 	const long long a_bytes = (long long)c->N * c->H * c->W * pixel_pitch * 2;
 	if (c->groups != 1 || c->C % 64 || M <= 0 || M > INT32_MAX || c->OC <= 0 ||
-	    a_bytes > 0x7FFFFFF0LL || (long long)c->OC * K1 * segs * 2 > 0x7FFFFFF0LL ||
+	    a_bytes > 0x7FFFFFF0LL || (long long)c->OC * K1 * (segs == 3 ? 2 : 1) * 2 > 0x7FFFFFF0LL ||
+	    (long long)K1 * segs > INT32_MAX ||
 	    (((uintptr_t)xa | (uintptr_t)wb) & 15u))
 		return (int)hipErrorInvalidValue;
 	ConvArgs q = {};
@@ -385,16 +387,18 @@ extern "C" int s3k_conv_implicit(const struct s3k_conv *c, const void *xa, const
 	q.g.M = (int)M;
 	q.g.N = c->OC;
 	q.g.K = K1 * segs;
-	q.g.ldb_b = (long long)K1 * segs * 2;
+	/* planes of K1, a multiple of 64: two per row */
+	q.g.kseg = segs == 3 ? K1 : 0;
+	q.g.ldb_b = (long long)K1 * (segs == 3 ? 2 : 1) * 2;
 	if (c->out_planes && (c->kind != S3K_F32 || c->OC % 8))
 		return (int)hipErrorInvalidValue;
-	q.g.ldc = c->out_planes ? 3 * c->OC : c->OC;
+	q.g.ldc = c->out_planes ? s3k_planes(c->OC) * c->OC : c->OC;
 	q.g.flags = c->flags & (S3K_EPI_BIAS | S3K_EPI_GELU);
 	q.g.c_kind = c->out_planes ? S3K_C_PLANES : c->kind;
 	q.g.bias_kind = c->kind;
 	q.g.vec_ok = (c->OC % 8 == 0) && (((uintptr_t)c->y & 15u) == 0);
 	q.g.a_extent = (unsigned)a_bytes;
-	q.g.b_extent = (unsigned)((long long)c->OC * K1 * segs * 2);
+	q.g.b_extent = (unsigned)((long long)c->OC * q.g.ldb_b);
 	q.H = c->H; q.W = c->W; q.C = c->C; q.KH = c->KH; q.KW = c->KW;
 	q.stride = c->stride; q.ph = c->pad_h; q.pw = c->pad_w; q.OH = c->OH; q.OW = c->OW;
 	q.PP = pixel_pitch;

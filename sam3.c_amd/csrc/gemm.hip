@@ -553,6 +553,7 @@ static GemmArgs make_args(const struct s3k_gemm *g)
 	p.qkv_dsh = g->qkv_D > 0 ? __builtin_ctz((unsigned)g->qkv_D) : 0;
 	p.qkv_rope = g->qkv_rope;
 	p.qkv_planes = g->qkv_planes;
+	p.kseg = g->kseg;
 	p.ps_s = g->ps_s;
 	p.ps_oc = g->ps_oc;
 	p.ps_w = g->ps_w;
@@ -709,6 +710,9 @@ extern "C" int s3k_gemm_launch_path(const struct s3k_gemm *g, int path, void *st
 	if ((g->flags & S3K_EPI_QKV) &&
 	    ((path != S3K_PATH_MFMA && path != S3K_PATH_SKINNY) ||
 	     (path == S3K_PATH_MFMA && !mfma_ok(g)) || !qkv_ok(g, path)))
+		return (int)hipErrorInvalidValue;
+	if (g->kseg && (g->kseg < 0 || g->kseg % 64 || g->K != 3LL * g->kseg || path != S3K_PATH_MFMA ||
+			g->batch != 1 || !s3k_dl_ok(g)))
 		return (int)hipErrorInvalidValue;
 	/* the pixel shuffle lives in the epilogue's unrolled store path: whole
 	 * wave tiles of columns, 16-byte rows, the direct-to-LDS kernels */

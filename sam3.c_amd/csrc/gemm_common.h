@@ -39,6 +39,7 @@ struct GemmArgs {
 	float *qkv_out[3];
 	const float *qkv_cos, *qkv_sin;
 	int qkv_S, qkv_H, qkv_dsh, qkv_rope, qkv_planes;
+	int kseg;              /* two planes per row (struct s3k_gemm), 0 = none */
 	int ps_s, ps_oc, ps_w; /* pixel shuffle (struct s3k_gemm), ps_s 0 = none */
 	int tstrip;   /* tile order (tile_of): 0, or N strips of this many tiles */
 	int xwalk;    /* each slice's tiles on one XCD: gemm_dlk 1; gemm_dlt the
@@ -99,6 +100,19 @@ __device__ __forceinline__ void mfma_chunk(s3k_f32x16 &acc, const uint4 &a, cons
 		acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.z), __uint_as_float(b.z), acc, 0, 0, 0);
 		acc = __builtin_amdgcn_mfma_f32_32x32x2f32(__uint_as_float(a.w), __uint_as_float(b.w), acc, 0, 0, 0);
 	}
+}
+
+/* Byte offset of k in a row of A or W: 2k, or its place in the two planes
+ * that k walks as hi, lo, hi (A) and hi, hi, lo (W). Steps never straddle
+ * a plane (kseg is a multiple of 64). */
+__device__ __forceinline__ unsigned k_off_a(const GemmArgs &p, int k)
+{
+	return 2u * (unsigned)(p.kseg && k >= 2 * p.kseg ? k - 2 * p.kseg : k);
+}
+
+__device__ __forceinline__ unsigned k_off_b(const GemmArgs &p, int k)
+{
+	return 2u * (unsigned)(p.kseg && k >= p.kseg ? k - p.kseg : k);
 }
 
 /* Workgroup id -> (tile_m, tile_n). Workgroups are dealt round-robin to
@@ -312,7 +326,8 @@ __device__ __forceinline__ float finishw(const GemmArgs &p, int flags, char *cb,
 		if (W == 8 && full && p.vec_ok) {
 			*(u4v *)c = (u4v){hi[0], hi[1], hi[2], hi[3]};
 			*(u4v *)(c + p.N) = (u4v){lo[0], lo[1], lo[2], lo[3]};
-			*(u4v *)(c + 2LL * p.N) = (u4v){hi[0], hi[1], hi[2], hi[3]};
+			if (p.N & 63)
+				*(u4v *)(c + 2LL * p.N) = (u4v){hi[0], hi[1], hi[2], hi[3]};
 		} else {
 #pragma unroll
 			for (int e = 0; e < W; ++e) {
@@ -322,7 +337,8 @@ __device__ __forceinline__ float finishw(const GemmArgs &p, int flags, char *cb,
 				const uint16_t l = (uint16_t)(e & 1 ? lo[e / 2] >> 16 : lo[e / 2] & 0xFFFFu);
 				c[e] = h;
 				c[p.N + e] = l;
-				c[2LL * p.N + e] = h;
+				if (p.N & 63)
+					c[2LL * p.N + e] = h;
 			}
 		}
 	} else if (CK == S3K_F32) {
@@ -683,7 +699,9 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 						*(s3k_u32x4 *)c = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
 						if constexpr (CK == S3K_C_PLANES) {
 							*(s3k_u32x4 *)(c + plane) = (s3k_u32x4){lo[0], lo[1], lo[2], lo[3]};
-							*(s3k_u32x4 *)(c + 2LL * plane) = (s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
+							if (plane & 63) /* s3k_planes */
+								*(s3k_u32x4 *)(c + 2LL * plane) =
+									(s3k_u32x4){hi[0], hi[1], hi[2], hi[3]};
 						}
 					}
 				} else if (m < p.M) {

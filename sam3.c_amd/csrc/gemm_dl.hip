@@ -102,10 +102,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dl(GemmArgs p)
 		if (k0 + BK <= p.K) {
 #pragma unroll
 			for (int j = 0; j < A_PER; ++j)
-				dma16s(st + j * NW * 1024, ra, a_off[j], 2u * k0);
+				dma16s(st + j * NW * 1024, ra, a_off[j], k_off_a(p, k0));
 #pragma unroll
 			for (int j = 0; j < B_PER; ++j)
-				dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], 2u * k0);
+				dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b(p, k0));
 		} else {
 #pragma unroll
 			for (int j = 0; j < A_PER; ++j) {
@@ -245,10 +245,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 1) gemm_dlp(GemmArgs p)
 	auto dma = [&](int kt, int t, int stg) {
 		if (t < A_PER)
 			dma16s(lds0 + (unsigned)(stg * A_BYTES + (t * NW + wave) * 1024), ra, off[t],
-			       (unsigned)(kt * BK * 2));
+			       k_off_a(p, kt * BK));
 		else
 			dma16s(lds0 + (unsigned)(B_BASE + stg * B_BYTES + ((t - A_PER) * NW + wave) * 1024),
-			       rb, off[t], (unsigned)(kt * BK * 2));
+			       rb, off[t], k_off_b(p, kt * BK));
 	};
 
 	unsigned abase[4], bbase[4];

@@ -23,11 +23,21 @@ enum s3k_kind {
 	S3K_BF16 = 2,
 	S3K_Q8   = 5,
 	/* output kinds only: f32 epilogue math, then the form the next GEMM
-	 * reads: f16 [M, ldc], or bf16 planes [hi|lo|hi] with row pitch
-	 * ldc = 3N (hi at n, lo at N + n, hi again at 2N + n) */
+	 * reads: f16 [M, ldc], or bf16 planes with row pitch
+	 * ldc = s3k_planes(N) * N (hi at n, lo at N + n, and with three
+	 * planes hi again at 2N + n) */
 	S3K_C_F16OP  = 16,
 	S3K_C_PLANES = 17,
 };
+
+/* Planes per row of the split f32 GEMM's A, over K values: [hi|lo], or
+ * [hi|lo|hi] when K is no whole number of 64-k steps (then the GEMM reads
+ * the tripled k as it lies; with two planes it walks hi, lo, hi by k-step,
+ * struct s3k_gemm kseg). W has [hi|lo] or [hi|hi|lo]. */
+static inline int s3k_planes(int K)
+{
+	return K % 64 ? 3 : 2;
+}
 
 /* Epilogue / layout flags. */
 #define S3K_EPI_BIAS 1  /* out += bias[n] (bias has the output's kind)    */
@@ -88,6 +98,10 @@ struct s3k_gemm {
 	int         batch;
 	int         a_kind, b_kind, c_kind;
 	int         flags;
+	/* > 0: A and W are two planes [hi|lo] of kseg values per row (bf16, a
+	 * multiple of 64), K = 3 * kseg: k walks A's hi, lo, hi against W's
+	 * hi, hi, lo. Direct-to-LDS kernels, batch 1. */
+	int         kseg;
 	const void *res;                          /* S3K_EPI_RES: f32 [M, N] */
 	/* row map (rm_g > 0): C row m is stored (and its residual read) at
 	 * row ((a*rm_d2 + c)*rm_d1 + b)*rm_g + m % rm_g, where
@@ -230,8 +244,8 @@ int s3k_attn_path(int kind, const void *q, const void *k, const void *v, void *o
  * item, oh | BH): head b*oh + h, query q is stored at row b*Sq + q,
  * columns h*D.., of [BH/oh * Sq, oh*D], the permute (0,2,1,3) of
  * [BH/oh, oh, Sq, D]. oh = 0 keeps [BH, Sq, D]. ofmt (f32 on the MFMA kernel
- * only): 0 f32 rows, S3K_LN_PLANES bf16 planes [hi|lo|hi] with row pitch
- * 3*oh*D, S3K_LN_F16 f16 rows storing ovf_tag to *ovf (when set) as
+ * only): 0 f32 rows, S3K_LN_PLANES bf16 planes (s3k_planes) with row pitch
+ * s3k_planes * oh*D, S3K_LN_F16 f16 rows storing ovf_tag to *ovf (when set) as
  * s3k_permute_to does: the merged rows as a GEMM's operand.
  * kvp: K and V are prepared planes, each row of 64 f32 values replaced by
  * 256 bytes of bf16 hi[64] | lo[64], hi = bf16(x), lo = bf16(x - hi);
@@ -259,7 +273,7 @@ int s3k_attn_heads_path(int kind, const void *q, const void *k, const void *v, v
 int s3k_layernorm(int kind, const void *x, const void *gamma, const void *beta, void *out,
 		  long long rows, int cols, void *stream);
 /* f32 LayerNorm written as the operand a GEMM reads: bf16 planes
- * [rows, 3*cols] = [hi|lo|hi] (S3K_LN_PLANES, the split f32 GEMM's A) or
+ * [rows, s3k_planes * cols] (S3K_LN_PLANES, the split f32 GEMM's A) or
  * f16 [rows, cols] (S3K_LN_F16, the Q8 GEMM's A); the same values as
  * s3k_layernorm followed by s3k_split3_bf16 / s3k_cast_f16. For the f16
  * form, ovf (when not NULL) receives ovf_tag if a row's largest |y| lies

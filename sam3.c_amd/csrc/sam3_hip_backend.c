@@ -943,7 +943,7 @@ static enum sam3_error run_matmul(struct sam3_hip_backend *hb, const struct sam3
 		/* an f16 operand carries its row tags (two words per row) after
 		 * the data: zeroed when the allocation is new to this form, then
 		 * stamped with each eval's own tag */
-		const size_t dbytes = ((size_t)M * N * (o_fmt == S3H_A_PLANES ? 6 : 2) + 15) & ~(size_t)15;
+		const size_t dbytes = ((size_t)M * N * (o_fmt == S3H_A_PLANES ? 2 * s3k_planes(N) : 2) + 15) & ~(size_t)15;
 		const int f16 = o_fmt == S3H_A_F16;
 		int same = 0;
 		unsigned *rowf = NULL;
@@ -1418,7 +1418,7 @@ static enum sam3_error run_permute_as(struct sam3_hip_backend *hb, const struct 
 	enum sam3_error err = dev_in(hb, n->inputs[0], &dx);
 	if (err == SAM3_OK)
 		err = dev_out_fmt(hb, n->output,
-				  (size_t)s3h_nelems(n->output) * (fmt == S3H_A_PLANES ? 6 : 2), fmt, &dy,
+				  (size_t)s3h_nelems(n->output) * (fmt == S3H_A_PLANES ? 2 * s3k_planes(K) : 2), fmt, &dy,
 				  NULL);
 	if (err == SAM3_OK)
 		err = s3h_transpose_to(n, dx, dy, fmt, K, hb->ovf, hb->ovf_tag, hb->stream);
@@ -1494,7 +1494,7 @@ static enum sam3_error run_layernorm_map(struct sam3_hip_backend *hb, const stru
 	if (err == SAM3_OK && n->n_inputs > 2 && n->inputs[2])
 		err = dev_in(hb, n->inputs[2], &db);
 	if (err == SAM3_OK)
-		err = dev_out_fmt(hb, t, (size_t)rows * cols * (fmt == S3H_A_PLANES ? 6 : 2), fmt, &dy,
+		err = dev_out_fmt(hb, t, (size_t)rows * cols * (fmt == S3H_A_PLANES ? 2 * s3k_planes(cols) : 2), fmt, &dy,
 				  NULL);
 	if (err == SAM3_OK)
 		err = s3h_hip(s3k_layernorm_to_map(fmt == S3H_A_PLANES ? S3K_LN_PLANES : S3K_LN_F16,
@@ -1524,7 +1524,7 @@ static enum sam3_error run_layernorm_as(struct sam3_hip_backend *hb, const struc
 	if (err == SAM3_OK && n->n_inputs > 2 && n->inputs[2])
 		err = dev_in(hb, n->inputs[2], &db);
 	if (err == SAM3_OK)
-		err = dev_out_fmt(hb, n->output, (size_t)rows * cols * (fmt == S3H_A_PLANES ? 6 : 2),
+		err = dev_out_fmt(hb, n->output, (size_t)rows * cols * (fmt == S3H_A_PLANES ? 2 * s3k_planes(cols) : 2),
 				  fmt, &dy, NULL);
 	if (err == SAM3_OK)
 		err = s3h_hip(s3k_layernorm_to(fmt == S3H_A_PLANES ? S3K_LN_PLANES : S3K_LN_F16,
@@ -1633,7 +1633,7 @@ static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_g
 	/* a result only the next convolution reads: written as its planes */
 	const int out_planes = (transposed ? s3h_conv_transpose2d_planes(&dn) : s3h_conv2d_planes_out(&dn)) &&
 			       conv_planes_reader(hb, g, j, out, uses);
-	err = out_planes ? dev_out_fmt(hb, out, (size_t)ny * 6, S3H_A_PLANES, &ty.data, NULL)
+	err = out_planes ? dev_out_fmt(hb, out, (size_t)ny * 2 * s3k_planes(out->dims[3]), S3H_A_PLANES, &ty.data, NULL)
 			 : dev_out(hb, out, &ty.data);
 	if (err != SAM3_OK)
 		return err;
@@ -1789,7 +1789,7 @@ static enum sam3_error run_sdpa_merged(struct sam3_hip_backend *hb, const struct
 		err = dev_out(hb, t->output, &dy);
 	else
 		err = dev_out_fmt(hb, t->output,
-				  (size_t)s3h_nelems(t->output) * (fmt == S3H_A_PLANES ? 6 : 2), fmt, &dy,
+				  (size_t)s3h_nelems(t->output) * (fmt == S3H_A_PLANES ? 4 : 2), fmt, &dy,
 				  NULL);
 	if (err == SAM3_OK)
 		err = s3h_sdpa_merged(&dn, dy, fmt, hb->ovf, hb->ovf_tag, kvp, hb->stream);

@@ -93,8 +93,8 @@ int s3h_bias_add_ok(const struct sam3_node *node);
 enum sam3_error s3h_bias_add(const struct sam3_node *node, void *stream);
 
 /* The form matmul converts its A operand to before the GEMM, so the node
- * producing A can write that form directly: S3H_A_PLANES = bf16 [M, 3K]
- * [hi|lo|hi] (the split f32 GEMM), S3H_A_F16 = f16 [M, K] (the Q8 GEMM
+ * producing A can write that form directly: S3H_A_PLANES = bf16 planes
+ * of K, s3k_planes(K) per row (the split f32 GEMM), S3H_A_F16 = f16 [M, K] (the Q8 GEMM
  * with f32 activations). s3h_matmul_fmt runs the GEMM on A in that form. */
 enum { S3H_A_PLAIN = 0, S3H_A_PLANES = 1, S3H_A_F16 = 2, S3H_A_LN = 3, S3H_A_ATT1 = 4,
        S3H_KV_PLANES = 5 };
@@ -170,7 +170,8 @@ enum sam3_error s3h_matmul_qkv(int a_fmt, int a_dt, const void *a, int b_dt, con
  * to be constant (a mapped weight range, or an uploaded input that no
  * node writes), and dropped with that memory. Outside graph_eval nothing
  * is cached. */
-enum { S3H_PREP_SPLIT_W = 1,   /* f32 [rows, k] -> bf16 [rows, 3k] = [hi|hi|lo] */
+enum { S3H_PREP_SPLIT_W = 1,   /* f32 [rows, k] -> bf16 planes of W (s3k_planes(k) of
+				* them per row)                               */
        S3H_PREP_PAD_PLANES,    /* f32 [rows, K] -> bf16 [rows, 3k] over k >= K, zero padded */
        S3H_PREP_PAD16,         /* 16-bit [rows, K] -> [rows, k], zero padded */
        S3H_PREP_Q8_F16,        /* Q8_0 [rows, k] -> f16 [rows, k] (q*scale

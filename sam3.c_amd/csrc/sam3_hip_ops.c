@@ -762,10 +762,11 @@ static int q8_dl_wants_cast(const struct s3k_gemm *g)
 }
 
 /* f32 x f32 with W [N,K] on the bf16 MFMA GEMM: A and W are split once
- * into bf16 hi/lo planes laid out along a tripled k, A' = [Ah | Al | Ah]
- * and W' = [Wh | Wh | Wl], so that one bf16 GEMM over 3K accumulates
+ * into bf16 hi/lo planes that one bf16 GEMM walks along a tripled k,
+ * A' = [Ah | Al | Ah] against W' = [Wh | Wh | Wl], accumulating
  * Ah*Wh + Al*Wh + Ah*Wl in f32; the dropped Al*Wl term is below 2^-16 of
- * each product. */
+ * each product. Each plane is stored once when K is a multiple of 64
+ * (s3k_planes): 4 bytes per value to write and read instead of 6. */
 static int f32_split_wanted(const struct s3k_gemm *g)
 {
 	if (!s3h_settings()->f32_split)
@@ -778,11 +779,12 @@ static int f32_split_wanted(const struct s3k_gemm *g)
 	       (long long)g->M * g->N * g->K >= (1LL << 24);
 }
 
-/* a_planes: A already split by its producer ([M, 3K] = [hi|lo|hi]), or
- * NULL to split g->a here. */
+/* a_planes: A already split by its producer (s3k_planes(K) planes per
+ * row), or NULL to split g->a here. */
 static enum sam3_error f32_split_gemm(const struct s3k_gemm *g, const void *a_planes, void *stream)
 {
-	const size_t abytes = (size_t)g->M * 3 * g->K * 2, bbytes = (size_t)g->N * 3 * g->K * 2;
+	const int np = s3k_planes(g->K);
+	const size_t abytes = (size_t)g->M * np * g->K * 2, bbytes = (size_t)g->N * np * g->K * 2;
 	void *a3 = NULL, *b3 = NULL;
 	int own_b = 1;
 	enum sam3_error err = SAM3_OK;
@@ -807,7 +809,8 @@ static enum sam3_error f32_split_gemm(const struct s3k_gemm *g, const void *a_pl
 		h.b = b3;
 		h.a_kind = h.b_kind = S3K_BF16;
 		h.K = 3 * g->K;
-		h.lda = h.ldb = 3 * g->K;
+		h.lda = h.ldb = np * g->K;
+		h.kseg = np == 2 ? g->K : 0;
 		err = s3h_hip(s3k_gemm_launch_path(&h, S3K_PATH_MFMA, stream), "matmul f32 split gemm");
 	}
 	enum sam3_error ferr = SAM3_OK;
@@ -1060,7 +1063,7 @@ int s3h_matmul_out_ok(int a_fmt, int a_dt, const void *a, int b_dt, const void *
 			return 0;
 		h.a_kind = h.b_kind = S3K_BF16;
 		h.K = 3 * K;
-		h.lda = h.ldb = 3 * K;
+		h.lda = h.ldb = s3k_planes(K) * K;
 		return s3k_dl_eligible(&h);
 	}
 	if (b_dt != SAM3_DTYPE_Q8_0 || a_fmt != S3H_A_F16 || a_dt != SAM3_DTYPE_F32)
@@ -1124,7 +1127,7 @@ int s3h_matmul_res_ok(int a_fmt, int a_dt, const void *a, int b_dt, const void *
 }
 
 /* The GEMM of s3h_matmul_fmt with its f32 result written as out_fmt:
- * bf16 planes [M, 3N] = [hi|lo|hi] per row, or f16 [M, N], with the
+ * bf16 planes (s3k_planes(N) per row), or f16 [M, N], with the
  * bias and GELU applied in f32 first, the values split3 / the f16 cast
  * of the f32 output would give. */
 enum sam3_error s3h_matmul_fmt_to(int a_fmt, int out_fmt, int a_dt, const void *a, int b_dt,
@@ -1148,7 +1151,7 @@ enum sam3_error s3h_matmul_fmt_to(int a_fmt, int out_fmt, int a_dt, const void *
 	g.c_kind = out_fmt == S3H_A_PLANES ? S3K_C_PLANES
 		 : out_fmt == S3H_A_F16     ? S3K_C_F16OP
 					    : S3K_F32;
-	g.ldc = out_fmt == S3H_A_PLANES ? 3 * N : N;
+	g.ldc = out_fmt == S3H_A_PLANES ? s3k_planes(N) * N : N;
 	if (out_fmt == S3H_A_F16) {
 		g.ovf = ovf;
 		g.ovf_tag = ovf_tag;
@@ -2153,11 +2156,12 @@ static int conv_implicit_ok(const struct s3k_conv *c)
 {
 	const int f32 = c->kind == SAM3_DTYPE_F32;
 	const long long K = (long long)c->KH * c->KW * c->C;
-	const long long pp = f32 ? 3LL * c->C : c->C;
+	const long long pp = f32 ? 2LL * c->C : c->C;
 	return c->groups == 1 && (!f32 || conv_f32_split_allowed()) && c->C % 64 == 0 &&
 	       !(((uintptr_t)c->x | (uintptr_t)c->w) & 15u) &&
 	       (long long)c->N * c->H * c->W * pp * 2 <= 0x7FFFFFF0LL &&
-	       (long long)c->OC * K * (f32 ? 3 : 1) * 2 <= 0x7FFFFFF0LL;
+	       (long long)c->OC * K * (f32 ? 2 : 1) * 2 <= 0x7FFFFFF0LL &&
+	       (!f32 || 3 * K <= 0x7FFFFFF0LL);
 }
 
 static int conv_im2col_ok(const struct s3k_conv *c)
@@ -2211,15 +2215,15 @@ static enum sam3_error conv_run(struct s3k_conv *c, int path, int x_planes, void
 		void *xp = NULL, *wp = NULL;
 		int own_w = 0;
 		if (!x_planes)
-			err = s3h_scratch_alloc(&xp, (size_t)pix * 3 * c->C * 2, stream);
+			err = s3h_scratch_alloc(&xp, (size_t)pix * 2 * c->C * 2, stream);
 		if (err == SAM3_OK)
 			err = prep_weight(c->w, (size_t)c->OC * K * 4, S3H_PREP_SPLIT_W, c->OC, K, K,
-					  (size_t)c->OC * 3 * K * 2, S3K_F32, prep_split_w, stream, &wp, &own_w);
+					  (size_t)c->OC * 2 * K * 2, S3K_F32, prep_split_w, stream, &wp, &own_w);
 		if (err == SAM3_OK && !x_planes)
 			err = s3h_hip(s3k_split3_bf16((const float *)c->x, xp, (int)pix, c->C, c->C, 0, stream),
 				      "conv2d split x");
 		if (err == SAM3_OK)
-			err = s3h_hip(s3k_conv_implicit(c, x_planes ? c->x : xp, wp, 3 * c->C, stream),
+			err = s3h_hip(s3k_conv_implicit(c, x_planes ? c->x : xp, wp, 2 * c->C, stream),
 				      "conv2d implicit");
 		return free_scratch(xp, stream, free_scratch(own_w ? wp : NULL, stream, err));
 	}
@@ -2522,7 +2526,7 @@ enum sam3_error s3h_conv_transpose2d(const struct sam3_node *node, const void *b
 	if (err == SAM3_OK && convt_shuffle_gemm(&c, wt, bias, flags, &sg)) {
 		if (out_planes) {
 			sg.c_kind = S3K_C_PLANES;
-			sg.ldc = 3 * c.OC;
+			sg.ldc = 2 * c.OC; /* s3k_planes of a multiple of 64 */
 		} else {
 			sg.ldc = c.OC;
 		}
