@@ -656,7 +656,7 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 			for (int it = 0; it < IT; ++it) {
 				const int s = lane + 64 * it;
 				const int m = m0 + i * 32 + s / (WTN / W), n = n0 + (s % (WTN / W)) * W;
-				if constexpr (EB || EG) {
+				if constexpr ((EB || EG) && CK != S3K_BF16 && CK != S3K_F16) {
 #pragma unroll
 					for (int e = 0; e < W; ++e)
 						v[it][e] = epilogue<CK>(v[it][e], ein.b[e], (EB ? S3K_EPI_BIAS : 0) |
@@ -722,8 +722,8 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 						uint32_t w[4];
 #pragma unroll
 						for (int e = 0; e < 4; ++e)
-							w[e] = CK == S3K_BF16 ? pack_bf16x2(v[it][2 * e], v[it][2 * e + 1])
-									      : pack_f16x2(v[it][2 * e], v[it][2 * e + 1]);
+							w[e] = epilogue2<CK, EB, EG>(v[it][2 * e], v[it][2 * e + 1],
+										     ein.b[2 * e], ein.b[2 * e + 1]);
 						__builtin_nontemporal_store((s3k_u32x4){w[0], w[1], w[2], w[3]},
 									    (s3k_u32x4 *)((uint16_t *)cb + o));
 					}

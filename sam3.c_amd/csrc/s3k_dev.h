@@ -231,6 +231,7 @@ __device__ __forceinline__ float gelu_tanh(float x)
 }
 
 typedef __bf16 s3k_bf16x2 __attribute__((ext_vector_type(2)));
+typedef _Float16 s3k_f16x2 __attribute__((ext_vector_type(2)));
 typedef float s3k_f32x2 __attribute__((ext_vector_type(2)));
 
 /* Pack two f32 as two bf16 (RNE, NaN stays NaN) in one dword, lo first:
@@ -256,10 +257,12 @@ __device__ __forceinline__ float round_bf16_hw(float f)
 	return __uint_as_float(pack_bf16x2(f, 0.0f) << 16);
 }
 
-/* Pack two f32 as two f16 (RNE) in one dword, lo first. */
+/* Pack two f32 as two f16 (RNE) in one dword, lo first: one
+ * v_cvt_pk_f16_f32 on gfx950. */
 __device__ __forceinline__ uint32_t pack_f16x2(float lo, float hi)
 {
-	return f32_to_f16(lo) | (f32_to_f16(hi) << 16);
+	const s3k_f32x2 v = {lo, hi};
+	return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, s3k_f16x2));
 }
 
 /* Four signed bytes of w, each times s, as four f16 in two dwords. The
@@ -303,6 +306,33 @@ __device__ __forceinline__ float epilogue(float acc, float bias, int flags)
 			v = gelu_tanh(v);
 	}
 	return v;
+}
+
+/* epilogue<CK> of two neighbouring outputs of a 16-bit kind, packed. Each
+ * rounding is one conversion of the pair and the last one is the packed
+ * result, where value by value every rounding took a conversion of its own
+ * and the pack one more: about 3 (bf16) or 2 (f16) of 20 VALU instructions
+ * per output of an epilogue that nothing overlaps: 5184x4096x1024 bf16 with
+ * bias and GELU 53.9 -> 51.6 us. */
+template <int CK, bool BIAS, bool GELU>
+__device__ __forceinline__ uint32_t epilogue2(float x0, float x1, float b0, float b1)
+{
+	static_assert(CK == 1 || CK == 2, "16-bit kinds");
+	auto pack = [](float a, float b) { return CK == 2 ? pack_bf16x2(a, b) : pack_f16x2(a, b); };
+	uint32_t w = pack(x0, x1);
+	auto unpack = [&]() {
+		x0 = CK == 2 ? __uint_as_float(w << 16) : f16_to_f32(w & 0xFFFFu);
+		x1 = CK == 2 ? __uint_as_float(w & 0xFFFF0000u) : f16_to_f32(w >> 16);
+	};
+	if constexpr (BIAS) {
+		unpack();
+		w = pack(add_rn(x0, b0), add_rn(x1, b1));
+	}
+	if constexpr (GELU) {
+		unpack();
+		w = pack(gelu_tanh(x0), gelu_tanh(x1));
+	}
+	return w;
 }
 
 __device__ __forceinline__ float load_as_f32(const void *p, long long i, int kind)

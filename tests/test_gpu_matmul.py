@@ -636,6 +636,39 @@ def test_q8_gemv_f32_one_row(env, K, N):
     assert_f32_close(c16, refs[0], what="f16 stream")
 
 
+@pytest.mark.parametrize("kind", ["bf16", "f16"])
+@pytest.mark.parametrize("M,N,K", [(33, 72, 64), (300, 264, 192), (5184, 512, 64)])
+def test_16bit_epilogue_rounds_after_each_step(kind, M, N, K):
+    """Bias and GELU on 16-bit outputs, two at a time in the epilogue: the
+    result, the bias sum and the GELU each round once, so the fused outputs
+    are those of the plain product put through the same roundings (the
+    GELU's own exp and reciprocal may move a value to its neighbour)."""
+    import torch
+    dt, tt = (abi.BF16, torch.bfloat16) if kind == "bf16" else (abi.F16, torch.float16)
+    g = torch.Generator().manual_seed(763)
+    a = torch.randn(M, K, generator=g).to(tt).cuda()
+    w = (torch.randn(N, K, generator=g) * 0.2).to(tt).cuda()
+    bias = torch.randn(N, generator=g).to(tt).cuda()
+
+    def run(b, flags):
+        c = torch.empty(M, N, dtype=tt, device="cuda")
+        hip.matmul_dev(dt, a.data_ptr(), dt, w.data_ptr(), dt, c.data_ptr(), M, N, K, b, hip.B_NT | flags)
+        hip.synchronize()
+        return c
+
+    torch.cuda.synchronize()
+    plain = run(None, 0)
+    summed = run(bias.data_ptr(), hip.BIAS)
+    both = run(bias.data_ptr(), hip.BIAS | hip.GELU)
+    assert torch.equal(summed, (plain.float() + bias.float()).to(tt))
+    x = summed.double()
+    want = 0.5 * x * (1 + torch.tanh(0.7978845608 * (x + 0.044715 * x ** 3)))
+    # one rounding to the type (half an ulp) plus f32 arithmetic near it
+    eps = 2.0 ** -8 if kind == "bf16" else 2.0 ** -11
+    err = (both.double() - want).abs()
+    assert (err <= 1.01 * eps * want.abs() + 2.0 ** -20).all(), err.max()
+
+
 @pytest.mark.parametrize("K,N,B,shared", [(1024, 1024, 20, True), (4096, 1024, 5, False),
                                            (512, 256, 70, True), (512, 2048, 9, False),
                                            (1024, 2048, 20, True), (256, 256, 130, False),
