@@ -636,6 +636,32 @@ def test_q8_gemv_f32_one_row(env, K, N):
     assert_f32_close(c16, refs[0], what="f16 stream")
 
 
+@pytest.mark.parametrize("K,N", [(512, 4), (512, 1000), (1024, 1024), (1536, 36), (4096, 1024),
+                                 (4096, 4096), (4608, 64), (1024, 4100)])
+def test_q8_gemv_four_row_groups(env, K, N):
+    """One f32 row, K % 512 == 0 up to 4096, N % 4 == 0 up to 4096:
+    q8_gemv_rows4, the same bits as q8_gemv (which SAM3_HIP_SK_CFG=1,1
+    keeps, and which the sizes past either limit run anyway), within f32
+    rounding of the oracle's sums."""
+    O = oracle()
+    a, w, bias = rnd(760 + K, (1, K)), q8(rnd(761 + N, (N, K), 0.02)), rnd(762, N, 0.1)
+
+    def run():
+        plain = hip.matmul(a, abi.F32, w, abi.Q8_0, abi.F32, 1, N, K, flags=hip.B_NT)
+        full = hip.matmul(a, abi.F32, w, abi.Q8_0, abi.F32, 1, N, K, bias=bias,
+                          flags=hip.B_NT | hip.BIAS | hip.GELU)
+        return plain, full
+
+    got = run()
+    env.set("SAM3_HIP_SK_CFG", "1,1")
+    for x, y in zip(got, run()):
+        assert np.array_equal(x.view(np.uint32), y.view(np.uint32))
+    ref = ref_q8(a, w, K, N, nt=True)
+    assert np.max(np.abs(got[0] - ref)) <= 1e-5 * np.sqrt(K / 256) * np.max(np.abs(ref))
+    assert_f32_close(got[1], O.gelu(O.bias_add(ref, bias, "f32"), "f32").reshape(1, N),
+                     what="four-row groups, bias and GELU")
+
+
 @pytest.mark.parametrize("kind", ["bf16", "f16"])
 @pytest.mark.parametrize("M,N,K", [(33, 72, 64), (300, 264, 192), (5184, 512, 64)])
 def test_16bit_epilogue_rounds_after_each_step(kind, M, N, K):
