@@ -157,6 +157,12 @@ __global__ void __launch_bounds__(256) rowflag_check_k(RowFlagSet s, unsigned ta
 		*ovf = tag;
 }
 
+__global__ void word_copy_k(const unsigned *src, unsigned *dst)
+{
+	if (threadIdx.x == 0)
+		*dst = *src;
+}
+
 /* One thread per output of f16 [N,K]; element (n,k) reads block lin/32
  * of the flat Q8 array, lin = k*N+n (KN) or n*K+k (NK, rows that split
  * blocks), and is stored as f16(q * (scale / cs[n])). */
@@ -533,6 +539,12 @@ extern "C" int s3k_rowflag_check(int n, unsigned *const *flags, const int *rows,
 		return 0;
 	hipLaunchKernelGGL(rowflag_check_k, dim3((unsigned)((most + 255) / 256), (unsigned)n),
 			   dim3(256), 0, (hipStream_t)stream, s, tag, ovf);
+	return (int)hipGetLastError();
+}
+
+extern "C" int s3k_word_copy(const unsigned *src, unsigned *dst, void *stream)
+{
+	hipLaunchKernelGGL(word_copy_k, dim3(1), dim3(64), 0, (hipStream_t)stream, src, dst);
 	return (int)hipGetLastError();
 }
 

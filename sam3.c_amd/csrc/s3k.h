@@ -304,6 +304,8 @@ int s3k_permute_to(int fmt, const float *src, void *dst, int ndim, const int *in
  * below 2^-10. n <= 32 per call. */
 int s3k_rowflag_check(int n, unsigned *const *flags, const int *rows, unsigned tag, unsigned *ovf,
 		      void *stream);
+/* *dst = *src on the stream; dst may be pinned host memory. */
+int s3k_word_copy(const unsigned *src, unsigned *dst, void *stream);
 /* Whether the skinny launch of g rounds its f32 / bf16 activations to f16
  * with per-row power-of-two factors inside the kernel (no row-scaled f16
  * copy needed first). */

@@ -119,6 +119,7 @@ struct sam3_hip_backend {
 	 * writers set to this eval's tag when a value does not fit f16
 	 * (then the eval is redone without f16 operand forms) */
 	unsigned *ovf;
+	unsigned *ovf_host; /* pinned: the word as the host reads it */
 	unsigned ovf_tag;
 	int f16_writes;
 	int no_f16_ops;
@@ -1999,13 +2000,13 @@ static enum sam3_error hip_graph_eval(struct sam3_backend *be, struct sam3_graph
 	 * inputs are unchanged by the first run (nodes write only their own
 	 * outputs), so the second run starts from the same state. */
 	if (err == SAM3_OK && hb->f16_writes) {
-		unsigned tag = 0;
-		err = s3h_hip(hipMemcpyAsync(&tag, hb->ovf, sizeof(tag), hipMemcpyDeviceToHost,
-					     hb->stream),
-			      "graph_eval: range flag");
+		/* the flag reaches the host by a one-word kernel into pinned
+		 * memory: a copy call into pageable memory waits for the stream
+		 * and then copies */
+		err = s3h_hip(s3k_word_copy(hb->ovf, hb->ovf_host, hb->stream), "graph_eval: range flag");
 		if (err == SAM3_OK)
 			err = s3h_hip(hipStreamSynchronize(hb->stream), "graph_eval: range flag");
-		if (err == SAM3_OK && tag == hb->ovf_tag) {
+		if (err == SAM3_OK && *(volatile unsigned *)hb->ovf_host == hb->ovf_tag) {
 			const struct sam3_hip_eval_stats first = hb->stats;
 			memset(&hb->stats, 0, sizeof(hb->stats));
 			hb->stats.range_reruns = first.range_reruns + 1;
@@ -2099,6 +2100,9 @@ static enum sam3_error hip_init(struct sam3_backend *be)
 		err = s3h_hip(hipMalloc((void **)&hb->ovf, 256), "hip backend: range flag");
 	if (err == SAM3_OK)
 		err = s3h_hip(hipMemset(hb->ovf, 0, 256), "hip backend: range flag");
+	if (err == SAM3_OK)
+		err = s3h_hip(hipHostMalloc((void **)&hb->ovf_host, 256, hipHostMallocDefault),
+			      "hip backend: range flag");
 	return err;
 }
 
@@ -2145,6 +2149,10 @@ static void hip_free(struct sam3_backend *be)
 	if (hb->ovf) {
 		(void)hipFree(hb->ovf);
 		hb->ovf = NULL;
+	}
+	if (hb->ovf_host) {
+		(void)hipHostFree(hb->ovf_host);
+		hb->ovf_host = NULL;
 	}
 }
 
