@@ -371,8 +371,8 @@ __global__ void __launch_bounds__(256) permute_k(PermArgs a)
 }
 
 /* f32 permute whose last axis stays last, written as a GEMM operand: the
- * output, read as rows of K values, becomes bf16 planes [hi|lo|hi] with
- * row pitch 3K (PLANES) or f16 (else), the split / cast a GEMM applies
+ * output, read as rows of K values, becomes bf16 planes of K values
+ * per row (s3k_planes; PLANES) or f16 (else), the split / cast a GEMM applies
  * to f32 A. One thread per 4 values (one 16-byte source chunk). */
 template <bool PLANES, typename I>
 __global__ void __launch_bounds__(256) permute_op_k(PermArgs a, unsigned K)

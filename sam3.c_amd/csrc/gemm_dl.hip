@@ -943,7 +943,11 @@ extern "C" int s3k_dl_eligible(const struct s3k_gemm *g)
  *     13.6 here; 576x1024x4096 31.8 -> 20.2 (144 tiles), 169x768x3072
  *     24.9 -> 15.5 (36), 5184x512x512 8.1 -> 7.0 (648). Past 768 tiles
  *     the larger tiles' fewer L2 bytes win (2500x2048x512, 1280 tiles:
- *     10.7 here, 9.6 on 192x128);
+ *     10.7 here, 9.6 on 192x128). With K % 64 != 0 the line lies at 512:
+ *     rows then start off the 128-byte lines and the small tiles' larger
+ *     L2 traffic costs more (700x4096x1544, 704 tiles: 22.4 us here, 18.5
+ *     on 128x128; 2304x1024x2056 28.1 and 28.8; with K % 64 == 0
+ *     700x4096x2048 21.4 and 23.4);
  *   - 128x128 (cfg 4, 4 waves) between that and 192 tiles of 192x128.
  *   - K = 64 with M, N multiples of 192 and at least 1024 such tiles
  *     (attention scores over many slices): the persistent gemm_dlk,
@@ -966,7 +970,7 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 		const long long t9 = dl_tiles(g, 256, 256), t10 = dl_tiles(g, 192, 128);
 		const bool pipe = g->K % 64 == 0;
 		const long long t5 = dl_tiles(g, 64, 64);
-		if (t5 <= 768)
+		if (t5 <= (pipe ? 768 : 512))
 			cfg = t5 <= 512 ? 5 : 14;
 		else if (pipe && g->N <= 128 && t10 >= 192)
 			cfg = 24; /* narrow N: wider tiles would only compute padding */
@@ -986,8 +990,10 @@ int s3k_dl_launch(const struct s3k_gemm *g, GemmArgs p, hipStream_t st)
 	 * tile */
 	if ((g->flags & S3K_EPI_QKV) && (cfg < 20 || cfg == 25))
 		cfg = 26;
-	if (g->ps_s && cfg == 25) /* 96-column wave tiles: not the unrolled stores */
-		cfg = 24;
+	/* the pixel shuffle needs wave tiles of 32 or 64 columns, which every
+	 * N here divides by: not 96 (cfg 25), nor 128 (cfg 3, by setting only) */
+	if (g->ps_s && (cfg == 25 || cfg == 3))
+		cfg = cfg == 25 ? 24 : 10;
 	if ((s3h_settings()->dl_cfg < 0 || cfg == 30) && !g->ps_s && dlk_ok(g))
 		return g->a_kind == S3K_BF16 ? launch_dlk<FAM_BF16, 3>(g, p, st)
 					     : launch_dlk<FAM_F16, 3>(g, p, st);

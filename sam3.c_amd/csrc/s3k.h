@@ -143,6 +143,9 @@ struct s3k_gemm {
 	 * >= 4, qkv_S >= 32, N = E, 2E or 3E, M a multiple of qkv_S. When
 	 * bit y of qkv_planes is set (qkv_D = 64, not the skinny kernel),
 	 * each row of operand y is stored as planes (s3k_attn_heads, kvp). */
+	float       *qkv_out[3];
+	const float *qkv_cos, *qkv_sin;
+	int          qkv_S, qkv_H, qkv_D, qkv_rope, qkv_planes;
 	/* pixel shuffle (ps_s > 0): a transposed convolution with stride =
 	 * kernel = ps_s, N = ps_s^2 taps x ps_oc channels, row m the pixel
 	 * (m / ps_w, m % ps_w): column n, tap (kh, kw) = divmod(n / ps_oc,
@@ -151,9 +154,6 @@ struct s3k_gemm {
 	 * ldc and the planes' distance are those of ps_oc columns. ps_oc a
 	 * multiple of 64, direct-to-LDS GEMM, f32 or S3K_C_PLANES output */
 	int          ps_s, ps_oc, ps_w;
-	float       *qkv_out[3];
-	const float *qkv_cos, *qkv_sin;
-	int          qkv_S, qkv_H, qkv_D, qkv_rope, qkv_planes;
 };
 
 /* Which kernel s3k_gemm_launch would pick (for tests and the bench). */
@@ -293,7 +293,7 @@ int s3k_permute(int esize, const void *src, void *dst, int ndim, const int *in_d
 		const int *axes, void *stream);
 /* f32 permute (last axis kept, its size % 4 == 0) written as the operand
  * of a GEMM that reads the output as rows of K values: fmt S3K_LN_PLANES
- * (bf16 [hi|lo|hi], row pitch 3K) or S3K_LN_F16 (ovf as for
+ * (bf16, s3k_planes(K) per row) or S3K_LN_F16 (ovf as for
  * s3k_layernorm_to, checked per 4 values: one past 2^15, or all nonzero
  * and below 2^-10). */
 int s3k_permute_to(int fmt, const float *src, void *dst, int ndim, const int *in_dims,
@@ -345,9 +345,9 @@ int s3k_gelu(int kind, const void *x, void *out, long long n, void *stream);
  * y [N,OH,OW,OC], one kind for x, w, y (and bias, [OC], with
  * S3K_EPI_BIAS; S3K_EPI_GELU after it).
  *   s3k_conv_implicit: groups 1, C % 64 == 0; xa/wb are x and w for
- *     16-bit kinds, or their bf16 planes for f32 (x: [N*H*W, 3C] =
- *     [hi|lo|hi], w: [OC, 3K] = [hi|hi|lo], from s3k_split3_bf16);
- *     pixel_pitch = C or 3C.
+ *     16-bit kinds, or their bf16 planes for f32 (x: [N*H*W, 2C], w:
+ *     [OC, 2K], both [hi|lo], from s3k_split3_bf16); pixel_pitch = C
+ *     or 2C.
  *   s3k_conv_im2col: the column matrix [M, Kp] (16-bit) or its f32 planes
  *     [M, 3Kp] for the GEMM, Kp >= KH*KW*C, Kp % 8 == 0 (zero padded);
  *     s3k_conv_wprep: the weight as [OC, Kp] or planes [OC, 3Kp].

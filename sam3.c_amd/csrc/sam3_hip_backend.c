@@ -1542,9 +1542,6 @@ static enum sam3_error run_layernorm_as(struct sam3_hip_backend *hb, const struc
 	return err;
 }
 
-/* CONV2D or CONV_TRANSPOSE2D at node i, plus a following BIAS_ADD ([OC],
- * used only there) and GELU folded into the GEMM epilogue when the conv
- * runs as a GEMM. */
 /* Whether the f32 result `out` of the (transposed) convolution folded up to
  * node j may be written as bf16 planes: one node reads it (under any
  * header), a (transposed) convolution taking it as its input planes, whose
@@ -1586,6 +1583,9 @@ static int conv_planes_reader(struct sam3_hip_backend *hb, const struct sam3_gra
 	return n->op == SAM3_OP_CONV2D ? s3h_conv2d_planes_in(&dn) : s3h_conv_transpose2d_planes(&dn);
 }
 
+/* CONV2D or CONV_TRANSPOSE2D at node i, plus a following BIAS_ADD ([OC],
+ * used only there) and GELU folded into the GEMM epilogue when the conv
+ * runs as a GEMM. */
 static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_graph *g, int i,
 				struct use_map *uses, int *used)
 {
@@ -1649,8 +1649,6 @@ static enum sam3_error run_conv(struct sam3_hip_backend *hb, const struct sam3_g
 	return err;
 }
 
-/* ADD, GELU, TRANSPOSE, SDPA, LAYERNORM, ROPE, SLICE on device copies of
- * the node's tensors. */
 /* K and V of this SDPA node hold planes (kv_planes_fit) */
 static int kv_in_planes(struct sam3_hip_backend *hb, const struct sam3_node *n)
 {
@@ -1658,6 +1656,8 @@ static int kv_in_planes(struct sam3_hip_backend *hb, const struct sam3_node *n)
 	return k && k->fmt == S3H_KV_PLANES;
 }
 
+/* ADD, GELU, TRANSPOSE, SDPA, LAYERNORM, ROPE, SLICE on device copies of
+ * the node's tensors. */
 static enum sam3_error run_elementwise(struct sam3_hip_backend *hb, const struct sam3_node *n)
 {
 	struct sam3_tensor tin[SAM3_NODE_MAX_INPUTS], tout;
