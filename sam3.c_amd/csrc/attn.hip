@@ -175,8 +175,8 @@ struct at_int {
 };
 
 /* The probabilities of half a tile are formed against the running max m
- * without first taking the half's max: they are only recomputed (after
- * moving m to the half's max and rescaling the accumulators) when some
+ * without first taking the tile's max: they are only recomputed (after
+ * moving m to the tile's max and rescaling the accumulators) when some
  * lane's 32 probabilities sum past 2^15, which also catches the first
  * tile (m = -FLT_MAX gives +inf). Every probability the MFMA sees is
  * then below 2^15, inside the f16 range. */
@@ -585,13 +585,26 @@ __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_f
 				return ts;
 			};
 			/* if some lane's sum passed the bound: move the max to the
-			 * half's, rescale what is accumulated, redo half mb (rare) */
+			 * tile's, rescale what is accumulated, redo half mb (rare).
+			 * The scores of half 1 are still raw in settle(0): with a mask,
+			 * or keys past Sk in the tile, each half takes its own max, as
+			 * the raw score of a key that does not count could raise the
+			 * max until every real probability is 0. (Finishing half 1
+			 * before settle(0) takes 162 registers instead of 120; in a
+			 * copy inside it, 400 heads of 49 bf16 tokens take 5.9 us
+			 * instead of 5.4.) */
+			const bool whole = !MASK && kbase + AT_BKV <= p.Sk;
 			auto settle = [&](int mb, float ts) {
 				if (__builtin_amdgcn_ballot_w64(!(ts <= AT_PSUM_MAX))) {
 					float mt = s[mb][0];
 #pragma unroll
 					for (int r = 1; r < 16; ++r)
 						mt = fmaxf(mt, s[mb][r]);
+					if (whole) {
+#pragma unroll
+						for (int r = 0; r < 16; ++r)
+							mt = fmaxf(mt, s[1 - mb][r]);
+					}
 					const float m_new = fmaxf(m_run, at_max_pair(mt) * LOG2E);
 					const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 					m_run = m_new;
@@ -898,13 +911,20 @@ __global__ void __launch_bounds__(256 * KS, KS > 1 ? 1 : MASK ? 2 : 3) attn_plan
 			return ts;
 		};
 		/* as attn_fwd: when some lane's sum passed the bound, move the max
-		 * to the half's, rescale, redo half mb */
+		 * to the tile's (to the half's where attn_fwd does so, for the same
+		 * bits), rescale, redo half mb */
+		const bool whole = !MASK && kbase + AT_BKV <= p.Sk;
 		auto settle = [&](int mb, float ts) {
 			if (__builtin_amdgcn_ballot_w64(!(ts <= AT_PSUM_MAX))) {
 				float mt = s[mb][0];
 #pragma unroll
 				for (int r = 1; r < 16; ++r)
 					mt = fmaxf(mt, s[mb][r]);
+				if (whole) {
+#pragma unroll
+					for (int r = 0; r < 16; ++r)
+						mt = fmaxf(mt, s[1 - mb][r]);
+				}
 				const float m_new = fmaxf(m_run, at_max_pair(mt) * LOG2E);
 				const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 				m_run = m_new;

@@ -410,3 +410,31 @@ def test_sdpa_planes_nan_and_inf_scores(env):
         outs[use], _ = run(abi.F32, q, k, v, mask, path=MFMA)
     assert np.isnan(outs["1"][0, 3]).all() and np.isnan(outs["1"][:, 7]).all()
     assert np.array_equal(np.isnan(outs["0"]), np.isnan(outs["1"]))
+
+
+@pytest.mark.parametrize("dt", DTS, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("planes", ["0", "1"])
+def test_sdpa_max_is_of_scores_that_count(env, dt, planes):
+    """The running max is taken over keys that exist, with their mask: a
+    tile whose second half holds masked keys of raw score +200, or no keys
+    (raw score 0) beside real scores of -200, keeps its real
+    probabilities. Entries are multiples of 1/32 below 8, exact in bf16, so
+    the scores are exact too and the usual bounds hold."""
+    if dt != abi.F32 and planes == "1":
+        pytest.skip("planes are for f32")
+    env.set("SAM3_HIP_ATTN_PLANES", planes)
+    rng = np.random.default_rng(1295)
+    Sq, D = 40, 64
+    q = np.full((1, Sq, D), 5.0, np.float32)
+    v = synth.randn(1296, (1, 64, D))
+
+    k = -5.0 + rng.integers(-2, 3, (1, 40, D)).astype(np.float32) / 32
+    got, ref = run(dt, q, k, v[:, :40], path=MFMA)  # keys 40..63 of the tile do not exist
+    check(dt, got, ref, f"scores of -200, planes {planes}")
+
+    k = rng.integers(-2, 3, (1, 64, D)).astype(np.float32) / 32
+    k[:, 32:] += 5.0
+    mask = np.zeros((Sq, 64), np.float32)
+    mask[:, 32:] = -np.inf
+    got, ref = run(dt, q, k, v, mask, path=MFMA)
+    check(dt, got, ref, f"masked scores of +200, planes {planes}")
