@@ -120,7 +120,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) conv_dl(ConvArgs q)
 		}
 #pragma unroll
 		for (int j = 0; j < B_PER; ++j)
-			dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b(p, k0));
+			dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b<split_f32<FAM, CK>()>(p, k0));
 		w_ic += BK;
 		if (w_ic == q.C) {
 			w_ic = 0;

@@ -711,8 +711,11 @@ extern "C" int s3k_gemm_launch_path(const struct s3k_gemm *g, int path, void *st
 	    ((path != S3K_PATH_MFMA && path != S3K_PATH_SKINNY) ||
 	     (path == S3K_PATH_MFMA && !mfma_ok(g)) || !qkv_ok(g, path)))
 		return (int)hipErrorInvalidValue;
+	/* the two planes, and the pixel shuffle below: kernels from bf16 to
+	 * f32 or planes only (split_f32) */
+	const bool split = g->a_kind == S3K_BF16 && (g->c_kind == S3K_F32 || g->c_kind == S3K_C_PLANES);
 	if (g->kseg && (g->kseg < 0 || g->kseg % 64 || g->K != 3LL * g->kseg || path != S3K_PATH_MFMA ||
-			g->batch != 1 || !s3k_dl_ok(g)))
+			g->batch != 1 || !split || !s3k_dl_ok(g)))
 		return (int)hipErrorInvalidValue;
 	/* the pixel shuffle lives in the epilogue's unrolled store path: whole
 	 * wave tiles of columns, 16-byte rows, the direct-to-LDS kernels */
@@ -720,7 +723,7 @@ extern "C" int s3k_gemm_launch_path(const struct s3k_gemm *g, int path, void *st
 	    (g->ps_s < 0 || path != S3K_PATH_MFMA || !s3k_dl_ok(g) || g->batch != 1 || g->rm_g ||
 	     (g->flags & (S3K_EPI_RES | S3K_EPI_QKV)) || g->ps_oc <= 0 || g->ps_oc % 64 ||
 	     (long long)g->ps_s * g->ps_s * g->ps_oc != g->N || g->ps_w <= 0 || g->M % g->ps_w ||
-	     (g->c_kind != S3K_F32 && g->c_kind != S3K_C_PLANES) || !p.vec_ok))
+	     !split || !p.vec_ok))
 		return (int)hipErrorInvalidValue;
 	/* the weight-row factors: every MFMA GEMM rounding q*scale to f16
 	 * applies them (S3K_EPI_COLSCALE), and only the MFMA epilogue takes

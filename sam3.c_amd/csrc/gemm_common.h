@@ -102,17 +102,29 @@ __device__ __forceinline__ void mfma_chunk(s3k_f32x16 &acc, const uint4 &a, cons
 	}
 }
 
-/* Byte offset of k in a row of A or W: 2k, or its place in the two planes
- * that k walks as hi, lo, hi (A) and hi, hi, lo (W). Steps never straddle
- * a plane (kseg is a multiple of 64). */
-__device__ __forceinline__ unsigned k_off_a(const GemmArgs &p, int k)
+/* Whether a kernel of family FAM with output kind CK may run the split f32
+ * GEMM (struct s3k_gemm kseg, ps_*): bf16 planes to f32 or planes. The
+ * others are built without its offsets and its pixel shuffle: with them
+ * as run-time tests, bf16 5184x1024x136 took 6.55 us instead of 6.25. */
+template <int FAM, int CK>
+constexpr bool split_f32()
 {
-	return 2u * (unsigned)(p.kseg && k >= 2 * p.kseg ? k - 2 * p.kseg : k);
+	return FAM == FAM_BF16 && (CK == S3K_F32 || CK == S3K_C_PLANES);
 }
 
+/* Byte offset of k in a row of A or W: 2k, or (SEG) its place in the two
+ * planes that k walks as hi, lo, hi (A) and hi, hi, lo (W). Steps never
+ * straddle a plane (kseg is a multiple of 64). */
+template <bool SEG>
+__device__ __forceinline__ unsigned k_off_a(const GemmArgs &p, int k)
+{
+	return 2u * (unsigned)(SEG && p.kseg && k >= 2 * p.kseg ? k - 2 * p.kseg : k);
+}
+
+template <bool SEG>
 __device__ __forceinline__ unsigned k_off_b(const GemmArgs &p, int k)
 {
-	return 2u * (unsigned)(p.kseg && k >= p.kseg ? k - p.kseg : k);
+	return 2u * (unsigned)(SEG && p.kseg && k >= p.kseg ? k - p.kseg : k);
 }
 
 /* Workgroup id -> (tile_m, tile_n). Workgroups are dealt round-robin to
@@ -459,9 +471,11 @@ struct RowWalk {
  * its iterations reads the next iteration's staged values first.
  * RES_OK false: no unrolled residual path (the kernel's registers leave
  * no room for it, or it takes no residual).
+ * PS_OK: the pixel shuffle (struct s3k_gemm, ps_*) may be asked for.
  * QKV_OK (TR, f32 output): the S3K_EPI_QKV epilogue only, a kernel of
  * its own (the other paths' registers would not leave room for it). */
-template <int FM, int FN, int WTN, int CK, bool TR = false, bool QKV_OK = false, bool RES_OK = true>
+template <int FM, int FN, int WTN, int CK, bool TR = false, bool QKV_OK = false, bool RES_OK = true,
+	  bool PS_OK = false>
 __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&acc)[FM][FN],
 					      char *smem, int wave, int lane, int m0, int n0, int bz)
 {
@@ -579,7 +593,7 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 	if (FIXED && (flags & S3K_EPI_BIAS)) {
 		const int cw = (lane % (WTN / W)) * W;
 		if (n0 + cw < p.N)
-			epi_bias<W>(p, p.ps_s ? (n0 + cw) % p.ps_oc : n0 + cw, ein.b);
+			epi_bias<W>(p, PS_OK && p.ps_s ? (n0 + cw) % p.ps_oc : n0 + cw, ein.b);
 	}
 	/* staged values of unit s: row s / (WTN / W), columns cw.. cw + W - 1 */
 	auto staged = [&](int s, float (&x)[W]) {
@@ -617,7 +631,7 @@ __device__ __forceinline__ void write_tile_ck(const GemmArgs &p, s3k_f32x16 (&ac
 		constexpr int IT = UNITS / 64;
 		/* pixel shuffle: the lane's tap and channel are the same for the
 		 * whole tile, its pixel (py, px) steps by RPI rows per store */
-		constexpr bool PS_CK = FIXED && (CK == S3K_F32 || CK == S3K_C_PLANES);
+		constexpr bool PS_CK = PS_OK && FIXED && (CK == S3K_F32 || CK == S3K_C_PLANES);
 		constexpr int RPI = FIXED ? 64 / (WTN / W) : 1;
 		int py = 0, px = 0, ptap = 0, pcol = 0;
 		const int plane = PS_CK && p.ps_s ? p.ps_oc : p.N;

@@ -102,10 +102,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dl(GemmArgs p)
 		if (k0 + BK <= p.K) {
 #pragma unroll
 			for (int j = 0; j < A_PER; ++j)
-				dma16s(st + j * NW * 1024, ra, a_off[j], k_off_a(p, k0));
+				dma16s(st + j * NW * 1024, ra, a_off[j], k_off_a<split_f32<FAM, CK>()>(p, k0));
 #pragma unroll
 			for (int j = 0; j < B_PER; ++j)
-				dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b(p, k0));
+				dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b<split_f32<FAM, CK>()>(p, k0));
 		} else {
 #pragma unroll
 			for (int j = 0; j < A_PER; ++j) {
@@ -181,7 +181,8 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dl(GemmArgs p)
 	}
 
 	__syncthreads();
-	write_tile_ck<FM, FN, WTN, CK, true>(p, acc, smem, wave, lane, tm * BM + wm0, tn * BN + wn0, bz);
+	write_tile_ck<FM, FN, WTN, CK, true, false, true, split_f32<FAM, CK>()>(
+		p, acc, smem, wave, lane, tm * BM + wm0, tn * BN + wn0, bz);
 }
 
 /*
@@ -245,10 +246,10 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 1) gemm_dlp(GemmArgs p)
 	auto dma = [&](int kt, int t, int stg) {
 		if (t < A_PER)
 			dma16s(lds0 + (unsigned)(stg * A_BYTES + (t * NW + wave) * 1024), ra, off[t],
-			       k_off_a(p, kt * BK));
+			       k_off_a<split_f32<FAM, CK>()>(p, kt * BK));
 		else
 			dma16s(lds0 + (unsigned)(B_BASE + stg * B_BYTES + ((t - A_PER) * NW + wave) * 1024),
-			       rb, off[t], k_off_b(p, kt * BK));
+			       rb, off[t], k_off_b<split_f32<FAM, CK>()>(p, kt * BK));
 	};
 
 	unsigned abase[4], bbase[4];
@@ -353,7 +354,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 1) gemm_dlp(GemmArgs p)
 	step(kt & 1, kt, false, false);
 
 	__syncthreads();
-	write_tile_ck<FM, FN, WTN, CK, true, QKV>(p, acc, smem, wave, lane, tm * BM + wm0,
+	write_tile_ck<FM, FN, WTN, CK, true, QKV, true, split_f32<FAM, CK>()>(p, acc, smem, wave, lane, tm * BM + wm0,
 						 tn * BN + wn0, bz);
 }
 
