@@ -1503,14 +1503,28 @@ extern "C" int s3k_attn_planes_ok(const void *q, const void *k, const void *v, c
 }
 
 /* Whether f32 K and V as they are are worth making planes of first. The
- * pass over them costs their bytes twice (1296 x 576 keys: 115 us; never
- * under about 3 us); the gain grows with the query blocks that share them,
- * and with a mask or idle CUs (ap_groups) there is more to gain. One box,
- * attn_fwd against pass + attn_planes_fwd, heads x queries [x keys]:
- * 16 x 5184 (41 blocks) 400 -> 334 us, 64 x 1600 (13) 152 -> 154, 100 x
- * 1024 (8) 102 -> 108, 1296 x 576 (5) 431 -> 466; masked 16 x 1369 120 ->
- * 52, 200 x 400 98 -> 71, 1296 x 300 x 200 250 -> 184, 400 x 100 x 600 (1)
- * 72 -> 79, 16 x 256 16.1 -> 17.1. */
+ * pass over them is a launch (about 2 us) and their bytes twice; what it
+ * gains depends on how the workgroups of 128 queries fill the 256 CUs, two
+ * at a time on attn_fwd (one with a mask), three on attn_planes_fwd (two).
+ * Heads x queries x keys, attn_fwd against pass + attn_planes_fwd in us:
+ *   - no mask, key groups: the gain grows with the key tiles, the pass with
+ *     the heads. 14 x 100 x 500 19.2, 19.1; 28 x 100 x 500 19.2, 21.2; 16 x
+ *     700 x 700 25.7, 23.8; 28 x 100 x 700 24.9, 25.9; 50 x 128 x 1500 49.6,
+ *     45.4; 90 x 128 x 1500 49.5, 54.7; 16 x 1369 x 1369 47.0, 40.7;
+ *   - no mask, one group: a round of workgroups saved (513..768: one
+ *     instead of two) or a better filled chip (past 1024), if 17 query
+ *     blocks share the pass. 32 x 2300 x 300 (576) 32.5, 29.7; 40 x 2500 x
+ *     300 (800) 38.8, 41.5; 100 x 3000 x 300 (2400) 91.6, 86.9; 24 x 3000 x
+ *     300 (576) 32.0, 28.6; 16 x 2048 x 700 (256) 26.2, 28.7; 1296 x 576 x
+ *     576 (5 blocks a head) 431, 466; 16 x 5184 x 5184 (656) 400, 334;
+ *   - mask, two groups: by whole pairs of key tiles. 14 x 100 x 500 24.3,
+ *     23.7; 28 x 100 x 500 24.4, 25.9; 64 x 128 x 1024 56.7, 46.2; 200 x 128
+ *     x 1024 59.6, 67.8; 16 x 1369 x 1369 120, 51;
+ *   - mask, one group: past 256 workgroups attn_fwd needs a second round.
+ *     64 x 600 x 400 (320) 46.0, 38.7; 200 x 300 x 300 (600) 52.6, 48.2; 64
+ *     x 300 x 300 (192) 18.4, 24.7; 200 x 200 x 64 (400) 14.1, 14.5;
+ *   - mask rows that attn_fwd cannot load 16 bytes at a time: also below
+ *     that. 64 x 300 x 301 27.1, 24.7; 100 x 200 x 301 27.1, 27.6. */
 extern "C" size_t s3k_attn_planes_want(int path, int kind, const void *q, const void *k,
 				       const void *v, const void *mask, void *out, int BH, int Sq,
 				       int Sk, int D, int oh, int ofmt)
@@ -1520,10 +1534,24 @@ extern "C" size_t s3k_attn_planes_want(int path, int kind, const void *q, const 
 	    attn_heads_pick(path, kind, q, k, v, out, BH, Sq, Sk, D, oh, ofmt) != S3K_ATTN_MFMA ||
 	    !ap_fits(mask, Sq, Sk))
 		return 0;
-	const int nqb = (Sq + 127) / 128;
-	const long long tiles = (long long)BH * nqb * ((Sk + AT_BKV - 1) / AT_BKV);
-	const bool shared = mask ? nqb >= 2 && tiles >= 256 : nqb >= 16;
-	if (use < 0 && !shared && ap_groups(BH, Sq, Sk, mask != nullptr) == 1)
+	const long long nqb = (Sq + 127) / 128, nkt = (Sk + AT_BKV - 1) / AT_BKV, wgs = BH * nqb;
+	const bool groups = ap_groups(BH, Sq, Sk, mask != nullptr) > 1;
+	bool gain;
+	if (!mask && groups) {
+		gain = BH <= 60 && BH <= 4 * (nkt - 5);
+	} else if (!mask) {
+		gain = nqb >= 17 && wgs > 512 && (wgs <= 768 || wgs > 1024);
+	} else {
+		const bool vec = Sk % 4 == 0 && !((uintptr_t)mask & 15u);
+		const long long pairs = nkt / 2;
+		if (groups)
+			gain = !vec || pairs * pairs >= BH;
+		else if (wgs > 256)
+			gain = nqb >= 2 && nqb + nkt > 3;
+		else
+			gain = !vec && wgs * nkt >= 256 && nkt >= 3 && (nqb >= 3 || nkt >= 7);
+	}
+	if (use < 0 && !gain)
 		return 0;
 	return (size_t)BH * (size_t)Sk * AT_D * 4 * 2;
 }

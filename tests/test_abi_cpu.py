@@ -211,3 +211,45 @@ def test_no_oracle_in_product_path():
                 text = _strip_c_comments(text)
             for b in banned:
                 assert b not in text, (p, b)
+
+
+# (heads, queries, keys, mask) -> us of attn_fwd, us of the planes' pass +
+# attn_planes_fwd, one MI355X; the mask's rows are 16-byte aligned when keys % 4 == 0
+PLANES_TIMES = [
+    ((4, 2048, 64, False), 6.3, 8.3), ((1, 5184, 200, False), 12.0, 13.5),
+    ((16, 2100, 130, False), 14.6, 15.9), ((16, 2048, 700, False), 26.2, 28.8),
+    ((16, 3000, 200, False), 17.7, 18.5), ((32, 2300, 300, False), 32.5, 29.7),
+    ((16, 5184, 130, False), 24.1, 21.4), ((40, 2500, 600, False), 66.0, 68.7),
+    ((56, 2500, 600, False), 86.1, 80.9), ((48, 2048, 300, False), 34.5, 35.8),
+    ((64, 1369, 600, False), 56.4, 54.9), ((100, 3000, 300, False), 91.6, 86.9),
+    ((4, 400, 2000, False), 63.8, 44.5), ((16, 128, 512, False), 19.2, 19.5),
+    ((32, 300, 700, False), 25.1, 26.9), ((16, 700, 700, False), 25.7, 24.2),
+    ((64, 128, 1024, False), 34.7, 36.4), ((50, 128, 1500, False), 49.6, 45.4),
+    ((90, 250, 2000, False), 66.0, 71.1), ((16, 1369, 1369, False), 47.0, 40.7),
+    ((8, 600, 400, True), 23.0, 25.2), ((64, 300, 300, True), 18.4, 24.7),
+    ((64, 600, 130, True), 30.9, 20.5), ((200, 200, 64, True), 14.1, 14.7),
+    ((200, 300, 300, True), 52.6, 48.6), ((200, 128, 1024, True), 59.6, 67.9),
+    ((64, 128, 1024, True), 56.7, 46.5), ((14, 100, 500, True), 24.3, 23.7),
+    ((28, 100, 500, True), 24.4, 25.9), ((28, 100, 700, True), 32.0, 33.7),
+    ((28, 250, 900, True), 43.9, 41.8), ((16, 1369, 201, True), 22.1, 18.0),
+    ((64, 300, 301, True), 27.1, 24.7), ((100, 200, 301, True), 27.1, 27.7),
+    ((16, 1369, 63, True), 8.9, 9.7), ((16, 1369, 1369, True), 120.0, 51.0),
+]
+
+
+@pytest.mark.parametrize("case,plain,planes", PLANES_TIMES,
+                         ids=["x".join(map(str, c[0][:3])) + "-mask" * c[0][3] for c in PLANES_TIMES])
+def test_attention_planes_are_made_where_they_pay(env, case, plain, planes):
+    """s3k_attn_planes_want, the rule by which f32 attention makes planes of
+    K and V first, against measured times of both ways. Where the two lie
+    within 3 % of each other either answer is fine."""
+    env.unset("SAM3_HIP_ATTN_PLANES")
+    want = hip.load().s3k_attn_planes_want
+    want.restype = C.c_size_t
+    want.argtypes = [C.c_int] * 2 + [C.c_void_p] * 5 + [C.c_int] * 6
+    BH, Sq, Sk, mask = case
+    got = want(0, abi.F32, 1 << 20, 1 << 20, 1 << 20, (1 << 20) if mask else None, 1 << 20, BH, Sq,
+               Sk, 64, 0, 0)
+    if abs(plain - planes) > 0.03 * plain:
+        assert (got > 0) == (planes < plain)
+    assert got in (0, BH * Sk * 512)
