@@ -297,6 +297,13 @@ static int is_device_ptr(const void *p)
 	return attr.type == hipMemoryTypeDevice || attr.type == hipMemoryTypeManaged;
 }
 
+/* Whether t's data is memory of the caller's on the device, which nodes
+ * read and write in place. The table holds host memory only. */
+static int caller_device(struct sam3_hip_backend *hb, const struct sam3_tensor *t)
+{
+	return t->data && !res_find(hb, t->data) && is_device_ptr(t->data);
+}
+
 /* Device address of tensor t's data, uploading it if needed. */
 static enum sam3_error dev_in(struct sam3_hip_backend *hb, const struct sam3_tensor *t,
 			      void **out)
@@ -400,8 +407,6 @@ static enum sam3_error dev_out(struct sam3_hip_backend *hb, const struct sam3_te
 	return SAM3_OK;
 }
 
-/* A device buffer of nbytes for output t holding the operand form fmt of
- * the one GEMM that reads it: never downloaded, stale after the eval. */
 /* The row tags collected so far: rows whose nonzero values were all
  * below 2^-10 set the range flag (s3k_rowflag_check). */
 static enum sam3_error rowf_flush(struct sam3_hip_backend *hb)
@@ -415,7 +420,11 @@ static enum sam3_error rowf_flush(struct sam3_hip_backend *hb)
 	return err;
 }
 
-/* *same (when not NULL): the allocation held this operand form before
+/* A device buffer of nbytes for output t holding the operand form fmt of
+ * the one node that reads it: never downloaded, stale after the eval. Not
+ * for caller_device tensors: the entry made for one would stand between
+ * the caller's memory and every later graph that names it.
+ * *same (when not NULL): the allocation held this operand form before
  * (not new, not another form), so words past the data keep their
  * contents from earlier evals of this form. */
 static enum sam3_error dev_out_fmt(struct sam3_hip_backend *hb, const struct sam3_tensor *t,
@@ -663,9 +672,9 @@ static int qkv_epilogue_chains(const struct sam3_graph *g, int i, int j,
 /* Whether k and v, the second and third attention operands that the qkv
  * GEMM at node i stores, may be stored as planes (S3H_KV_PLANES): no node
  * but one f32 SDPA of head size 64 reads their data (under any header),
- * none writes it before that, and the SDPA's kernel takes planes. dq:
- * device address of q. */
-static int kv_planes_fit(const struct sam3_graph *g, int i,
+ * none writes it before that, they are not the caller's device memory, and
+ * the SDPA's kernel takes planes. dq: device address of q. */
+static int kv_planes_fit(struct sam3_hip_backend *hb, const struct sam3_graph *g, int i,
 			 const struct qkv_chain *cs, const void *dq, struct use_map *uses)
 {
 	static const char al[16] __attribute__((aligned(16)));
@@ -692,7 +701,8 @@ static int kv_planes_fit(const struct sam3_graph *g, int i,
 		    (same_data(o->output, kt) || same_data(o->output, vt)))
 			return 0;
 	}
-	return s3k_attn_planes_ok(dq, al, al, mask ? al : NULL, (void *)al, qt->dims[0] * qt->dims[1],
+	return !caller_device(hb, kt) && !caller_device(hb, vt) &&
+	       s3k_attn_planes_ok(dq, al, al, mask ? al : NULL, (void *)al, qt->dims[0] * qt->dims[1],
 				  qt->dims[2], kt->dims[2], 64, 0, 0);
 }
 
@@ -908,7 +918,7 @@ static enum sam3_error run_matmul(struct sam3_hip_backend *hb, const struct sam3
 		const struct sam3_tensor *ct = NULL, *st = NULL;
 		for (int y = 0; y < n_qkv && err == SAM3_OK; y++) {
 			void *dy = NULL;
-			if (y == 1 && n_qkv == 3 && kv_planes_fit(g, i, qcs, qkv.out[0], uses)) {
+			if (y == 1 && n_qkv == 3 && kv_planes_fit(hb, g, i, qcs, qkv.out[0], uses)) {
 				qkv.planes = 6;
 				if (!s3h_matmul_qkv_ok(a_fmt, a_dt, da, b_dt, db, M, N, K, flags, &qkv))
 					qkv.planes = 0;
@@ -1063,9 +1073,9 @@ static int find_gemm_reader(const struct sam3_graph *g, int i, int j, const stru
  * chain of nodes folded into it, the last of them before node j), can be
  * written: t must be used once, through RESHAPE views only, as the A of a
  * MATMUL that converts A before its GEMM (s3h_matmul_a_format), with
- * rows of row_len values (the producer's row length). The consumer's
- * weight is resolved (and uploaded) here to decide with its device
- * address. */
+ * rows of row_len values (the producer's row length), and not the
+ * caller's device memory. The consumer's weight is resolved (and
+ * uploaded) here to decide with its device address. */
 static int consumer_operand_form(struct sam3_hip_backend *hb, const struct sam3_graph *g, int i,
 				 int j, const struct sam3_tensor *t, int row_len,
 				 struct use_map *uses, int *k_out)
@@ -1081,7 +1091,9 @@ static int consumer_operand_form(struct sam3_hip_backend *hb, const struct sam3_
 	static const char aligned_a[16] __attribute__((aligned(16)));
 	const int f = s3h_matmul_a_format(SAM3_DTYPE_F32, aligned_a, r.w->dtype, db, SAM3_DTYPE_F32,
 					  r.M, r.N, r.K, r.nt ? SAM3_HIP_B_NT : 0);
-	return f == S3H_A_F16 && hb->no_f16_ops ? S3H_A_PLAIN : f;
+	if (f == S3H_A_PLAIN || (f == S3H_A_F16 && hb->no_f16_ops) || caller_device(hb, t))
+		return S3H_A_PLAIN;
+	return f;
 }
 
 /* The form an f32 LAYERNORM at node i writes: its consumer's operand. */
@@ -1140,7 +1152,8 @@ static int ln_gemv_form(struct sam3_hip_backend *hb, const struct sam3_graph *g,
 	ln->x = dx;
 	ln->gamma = dg;
 	ln->beta = dbt;
-	return s3h_matmul_ln_ok(r.w->dtype, dw, r.M, r.N, r.K, SAM3_HIP_B_NT, ln);
+	return s3h_matmul_ln_ok(r.w->dtype, dw, r.M, r.N, r.K, SAM3_HIP_B_NT, ln) &&
+	       !caller_device(hb, n->output);
 }
 
 /* LAYERNORM left to its consuming GEMM: the output's residency entry
@@ -1222,7 +1235,10 @@ static int sdpa_gemv_form(struct sam3_hip_backend *hb, const struct sam3_graph *
 	at->mask = dm;
 	at->scale = 1.0f / sqrtf((float)D);
 	at->D = D;
-	return s3h_matmul_att1_ok(r.w->dtype, dw, r.M, r.N, r.K, SAM3_HIP_B_NT, at) ? j : -1;
+	return s3h_matmul_att1_ok(r.w->dtype, dw, r.M, r.N, r.K, SAM3_HIP_B_NT, at) &&
+			       !caller_device(hb, t->output)
+		       ? j
+		       : -1;
 }
 
 /* SDPA (and its head-merge TRANSPOSE t) left to the consuming GEMV: t's
@@ -1545,7 +1561,8 @@ static enum sam3_error run_layernorm_as(struct sam3_hip_backend *hb, const struc
 /* Whether the f32 result `out` of the (transposed) convolution folded up to
  * node j may be written as bf16 planes: one node reads it (under any
  * header), a (transposed) convolution taking it as its input planes, whose
- * weight no node of the graph writes. */
+ * weight no node of the graph writes, and it is not the caller's device
+ * memory. */
 static int conv_planes_reader(struct sam3_hip_backend *hb, const struct sam3_graph *g, int j,
 			      const struct sam3_tensor *out, struct use_map *uses)
 {
@@ -1578,7 +1595,7 @@ static int conv_planes_reader(struct sam3_hip_backend *hb, const struct sam3_gra
 	dn.output = &ty;
 	/* the reader's own output address decides its path as well, and a
 	 * caller may have put it anywhere on the device */
-	if ((uintptr_t)n->output->data & 15u)
+	if (((uintptr_t)n->output->data & 15u) || caller_device(hb, out))
 		return 0;
 	return n->op == SAM3_OP_CONV2D ? s3h_conv2d_planes_in(&dn) : s3h_conv_transpose2d_planes(&dn);
 }

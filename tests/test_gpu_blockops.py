@@ -1032,8 +1032,8 @@ def test_block_epilogues_keep_the_bits_of_separate_nodes(env, wkind, grid, windo
     assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
-def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
-    """Output of one ViT block of width e, evaluated twice on one backend."""
+def small_vit_graph(wkind, grid, window, is_global, e=256, heads=4):
+    """One ViT block of width e: its graph and output tensor."""
     npos = grid * grid
     G = graph.Graph()
     x = G.tensor(abi.F32, (npos, e), synth.randn(1300, (npos, e)), ephemeral=1)
@@ -1051,7 +1051,13 @@ def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
          "fc2_w": w(11, (e, 2 * e), 0.05, True), "fc2_b": w(12, (e,), 0.02)}
     c, s_ = graph.rope_tables(grid if is_global else window, e // heads)
     tc, ts = G.tensor(abi.F32, c.shape, c), G.tensor(abi.F32, s_.shape, s_)
-    out = graph.vit_block(G, x, p, heads, grid, window, is_global, tc, ts)
+    return G, graph.vit_block(G, x, p, heads, grid, window, is_global, tc, ts)
+
+
+def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
+    """Output of one ViT block of width e, evaluated twice on one backend."""
+    npos = grid * grid
+    G, out = small_vit_graph(wkind, grid, window, is_global, e, heads)
     be = hip.Backend(0)
     try:
         res = []
@@ -1064,3 +1070,75 @@ def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
         be.close()
     assert np.array_equal(res[0], res[1])
     return res[0]
+
+
+def outputs_on_device(G, pick, offset=0):
+    """Moves the node outputs that pick(i, node) names into device buffers
+    of their own (offset bytes in), filled with NaN: [(tensor, buffer)]."""
+    moved = []
+    for i in range(G.g.n_nodes):
+        n = G.g.nodes[i]
+        if not pick(i, n):
+            continue
+        t = n.output.contents
+        elems = int(np.prod(list(t.dims)[:t.n_dims]))
+        buf = hip.DeviceBuffer.of(np.full(elems + 64, np.nan, np.float32))
+        t.data = buf.ptr + offset
+        moved.append((t, buf))
+    return moved
+
+
+def assert_device_outputs_live(be, moved):
+    """A later graph on the backend whose outputs are the same device
+    buffers writes them (no_readback: only the buffers can hold them)."""
+    G = graph.Graph()
+    a = synth.randn(1350, (1 << 20,))
+    for t, _ in moved:
+        dims = list(t.dims)[:t.n_dims]
+        elems = int(np.prod(dims))
+        x = G.tensor(abi.F32, dims, a[:elems].reshape(dims))
+        y = abi.make_tensor(abi.F32, dims, t.data, elems * 4)
+        G.keep.append(y)
+        G.node(abi.OP_ADD, [x, x], y)
+    G.g.no_readback = True
+    assert be.graph_eval(G.g) == abi.OK
+    for t, buf in moved:
+        elems = int(np.prod(list(t.dims)[:t.n_dims]))
+        off = (t.data - buf.ptr) // 4
+        got = buf.download(np.float32, (off + elems,))[off:]
+        assert np.array_equal(got, 2 * a[:elems])
+
+
+@pytest.mark.parametrize("grid,window,is_global", [(12, 6, False), (14, 14, True)])
+@pytest.mark.parametrize("wkind", ["f32", "q8"])
+def test_block_with_every_intermediate_in_device_memory(wkind, grid, window, is_global):
+    """A caller may put intermediates into device buffers of its own. They
+    are read and written there: no fold keeps one of them in a form of its
+    own behind its address. Q, K and V are whole after the eval, the output
+    is that of host intermediates (f32: the same bits; Q8_0: its f16
+    operands are then rounded with row factors), and a later graph that
+    writes one of the buffers reaches it."""
+    npos, e = grid * grid, 256
+    G0, out0 = small_vit_graph(wkind, grid, window, is_global)
+    G, out = small_vit_graph(wkind, grid, window, is_global)
+    last = G.g.n_nodes - 1
+    moved = outputs_on_device(G, lambda i, n: i != last and n.op != abi.OP_RESHAPE and
+                              n.output.contents.dtype == abi.F32)
+    assert len(moved) > 10
+    be = hip.Backend(0)
+    try:
+        assert be.graph_eval(G0.g) == abi.OK and be.graph_eval(G.g) == abi.OK
+        assert be.stats().host_nodes == 0
+        want, got = out_array(out0, (npos, e)), out_array(out, (npos, e))
+        if wkind == "f32":
+            assert np.array_equal(want.view(np.uint32), got.view(np.uint32))
+        else:
+            assert_f32_close(got, want, what="device intermediates")
+        sdpa = next(G.g.nodes[i] for i in range(last) if G.g.nodes[i].op == abi.OP_SDPA)
+        for k in range(3):
+            t = sdpa.inputs[k].contents
+            elems = int(np.prod(list(t.dims)[:t.n_dims]))
+            assert np.isfinite(hip.download_ptr(t.data, elems * 4, np.float32)).all()
+        assert_device_outputs_live(be, moved)
+    finally:
+        be.close()

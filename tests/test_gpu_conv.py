@@ -362,3 +362,47 @@ def test_conv_chain_writes_planes(env, h, w, dim, d):
     assert st.operand_writes == (3 if d % 64 == 0 else 2)
     assert np.array_equal(a.view(np.uint32), b.view(np.uint32))
     assert_f32_close(a, ref, what="conv chain")
+
+
+@pytest.mark.parametrize("first", ["conv", "convt"])
+def test_conv_chain_through_device_memory(first):
+    """The result between two convolutions in a device buffer of the
+    caller's: it holds the f32 result afterwards, and a later graph that
+    writes the buffer reaches it."""
+    from sam3_amd import graph
+    from test_gpu_blockops import assert_device_outputs_live, out_array, outputs_on_device
+    F = abi.F32
+    x = synth.randn(330, (1, 32, 32, 64))
+    w2 = synth.randn(332, (64, 3, 3, 64), 0.05)
+
+    def build():
+        G = graph.Graph()
+        tx = G.tensor(F, x.shape, x)
+        if first == "conv":
+            w1 = synth.randn(331, (64, 1, 1, 64), 0.1)
+            t = G.node(abi.OP_CONV2D, [tx, G.tensor(F, w1.shape, w1)], G.tensor(F, x.shape), (1, 0, 1, 0))
+        else:
+            w1 = synth.randn(331, (64, 2, 2, 64), 0.1)
+            t = G.node(abi.OP_CONV_TRANSPOSE2D, [tx, G.tensor(F, w1.shape, w1)],
+                       G.tensor(F, (1, 64, 64, 64)), (2, 0, 0, 0))
+        y = G.node(abi.OP_CONV2D, [t, G.tensor(F, w2.shape, w2)], G.tensor(F, list(t.dims)), (1, 1, 1, 0))
+        return G, t, y, w1
+
+    G0, _, y0, w1 = build()
+    G, t, y, _ = build()
+    moved = outputs_on_device(G, lambda i, n: i == 0)
+    be = hip.Backend(0)
+    try:
+        assert be.graph_eval(G0.g) == abi.OK
+        assert be.stats().operand_writes == 1  # host memory: the planes are used
+        assert be.graph_eval(G.g) == abi.OK
+        shape = tuple(list(t.dims))
+        got, want = out_array(y, shape), out_array(y0, shape)
+        assert np.array_equal(got.view(np.uint32), want.view(np.uint32))
+        O = oracle()
+        ref = O.conv2d(x, w1, 1, 0, kind="f32") if first == "conv" else O.conv_transpose2d(x, w1, 2, 0)
+        mid = moved[0][1].download(np.float32, shape)
+        assert_f32_close(mid, ref.reshape(shape), what="intermediate in device memory")
+        assert_device_outputs_live(be, moved)
+    finally:
+        be.close()
