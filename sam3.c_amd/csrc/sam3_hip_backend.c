@@ -304,6 +304,13 @@ static int caller_device(struct sam3_hip_backend *hb, const struct sam3_tensor *
 	return t->data && !res_find(hb, t->data) && is_device_ptr(t->data);
 }
 
+/* The same, at an address that is no multiple of 16 (this backend's own
+ * buffers are). */
+static int caller_unaligned(struct sam3_hip_backend *hb, const struct sam3_tensor *t)
+{
+	return ((uintptr_t)t->data & 15u) && caller_device(hb, t);
+}
+
 /* Device address of tensor t's data, uploading it if needed. */
 static enum sam3_error dev_in(struct sam3_hip_backend *hb, const struct sam3_tensor *t,
 			      void **out)
@@ -701,6 +708,13 @@ static int kv_planes_fit(struct sam3_hip_backend *hb, const struct sam3_graph *g
 		    (same_data(o->output, kt) || same_data(o->output, vt)))
 			return 0;
 	}
+	/* the kernel that reads planes writes 16-byte aligned rows: the SDPA's
+	 * output, or that of the TRANSPOSE its heads may be merged into
+	 * (sdpa_merge_target), can be the caller's device memory anywhere */
+	const int j = next_reader(g, s + 1, n->output);
+	const struct sam3_tensor *mt = j >= 0 && g->nodes[j].op == SAM3_OP_TRANSPOSE ? g->nodes[j].output : NULL;
+	if (caller_unaligned(hb, n->output) || (mt && caller_unaligned(hb, mt)))
+		return 0;
 	return !caller_device(hb, kt) && !caller_device(hb, vt) &&
 	       s3k_attn_planes_ok(dq, al, al, mask ? al : NULL, (void *)al, qt->dims[0] * qt->dims[1],
 				  qt->dims[2], kt->dims[2], 64, 0, 0);

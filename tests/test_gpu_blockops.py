@@ -1142,3 +1142,25 @@ def test_block_with_every_intermediate_in_device_memory(wkind, grid, window, is_
         assert_device_outputs_live(be, moved)
     finally:
         be.close()
+
+
+@pytest.mark.parametrize("merge", ["0", "1"])
+def test_attention_into_unaligned_device_memory(env, merge):
+    """K and V stay f32 when the attention's output, or the merged rows it
+    is stored as, is device memory of the caller's that only the any-size
+    kernel can write: a block with both 4 bytes off 16-byte alignment."""
+    env.set("SAM3_HIP_SDPA_MERGE", merge)
+    grid, e = 14, 256
+    G0, out0 = small_vit_graph("f32", grid, grid, True)
+    G, out = small_vit_graph("f32", grid, grid, True)
+    sd = next(i for i in range(G.g.n_nodes) if G.g.nodes[i].op == abi.OP_SDPA)
+    moved = outputs_on_device(G, lambda i, n: i in (sd, sd + 1), offset=4)
+    assert G.g.nodes[sd + 1].op == abi.OP_TRANSPOSE and len(moved) == 2
+    be = hip.Backend(0)
+    try:
+        assert be.graph_eval(G0.g) == abi.OK and be.graph_eval(G.g) == abi.OK
+        assert_f32_close(out_array(out, (grid * grid, e)), out_array(out0, (grid * grid, e)),
+                         what="unaligned attention output")
+        assert_device_outputs_live(be, moved)
+    finally:
+        be.close()
