@@ -42,7 +42,8 @@ enum sam3_error s3h_transpose_to(const struct sam3_node *node, const void *src, 
 				 int K, unsigned *ovf, unsigned ovf_tag, void *stream);
 /* Device scratch reused in stream order: a block given back with
  * s3h_scratch_free(p, stream) is handed out again only to requests on
- * that stream. s3h_scratch_release(stream) returns the stream's idle
+ * that stream (hipStreamPerThread: by the same thread, as each has its
+ * own). s3h_scratch_release(stream) returns the stream's idle
  * blocks to the runtime (after synchronizing it). */
 enum sam3_error s3h_scratch_alloc(void **p, size_t nbytes, void *stream);
 enum sam3_error s3h_scratch_free(void *p, void *stream);

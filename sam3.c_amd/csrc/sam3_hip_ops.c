@@ -19,6 +19,7 @@
 #include "s3k.h"
 
 #include <hip/hip_runtime_api.h>
+#include <limits.h>
 #include <pthread.h>
 #include <stdarg.h>
 #include <stdio.h>
@@ -55,7 +56,10 @@ enum sam3_error s3h_hip(int e, const char *what)
  * free list tagged with the device and the stream of its last use; a
  * later request on that same stream may take it at once, because every
  * kernel that used it was enqueued on that stream before the new user.
- * Blocks are never handed to another stream. Requests take the smallest
+ * Blocks are never handed to another stream. hipStreamPerThread is one
+ * handle for as many streams as there are threads, so its blocks carry the
+ * thread's number too (`owner`); when a thread ends, its idle ones are
+ * marked, and freed by the next call that has to allocate. Requests take the smallest
  * free block that fits and is at most twice the request (or 4 MiB
  * larger); otherwise a new block is allocated with hipMalloc, after
  * returning the idle blocks of the device to the runtime if the first
@@ -66,6 +70,7 @@ struct s3h_blk {
 	void *p;
 	size_t n;
 	void *stream;
+	unsigned owner; /* hipStreamPerThread: the thread's number; else 0 */
 	int dev;
 	int busy;
 };
@@ -81,6 +86,52 @@ static int *s3h_bix;
 static size_t s3h_bix_cap;
 static int s3h_bix_dirty;
 static pthread_mutex_t s3h_blk_lock = PTHREAD_MUTEX_INITIALIZER;
+#define S3H_OWNER_GONE UINT_MAX /* idle block of a thread that has ended */
+static int s3h_ngone;
+static unsigned s3h_threads; /* thread numbers given out */
+static pthread_key_t s3h_thread_key;
+static int s3h_thread_key_ok;
+static pthread_once_t s3h_thread_once = PTHREAD_ONCE_INIT;
+
+static void thread_gone(void *num)
+{
+	pthread_mutex_lock(&s3h_blk_lock);
+	for (int i = 0; i < s3h_nblks; i++)
+		if (!s3h_blks[i].busy && s3h_blks[i].owner == (unsigned)(uintptr_t)num) {
+			s3h_blks[i].owner = S3H_OWNER_GONE;
+			s3h_ngone++;
+		}
+	pthread_mutex_unlock(&s3h_blk_lock);
+}
+
+static void thread_key_make(void)
+{
+	s3h_thread_key_ok = pthread_key_create(&s3h_thread_key, thread_gone) == 0;
+}
+
+/* no thread may call into an unloaded library when it ends */
+__attribute__((destructor)) static void thread_key_drop(void)
+{
+	if (s3h_thread_key_ok)
+		(void)pthread_key_delete(s3h_thread_key);
+}
+
+/* The owner of blocks used on `stream` by this thread. Called with the
+ * lock held. Numbers are not reused. Without a key for them every call gets a
+ * new number: its blocks are not reused, which is safe. */
+static unsigned stream_owner(void *stream)
+{
+	if (stream != (void *)hipStreamPerThread)
+		return 0;
+	(void)pthread_once(&s3h_thread_once, thread_key_make);
+	unsigned num = s3h_thread_key_ok ? (unsigned)(uintptr_t)pthread_getspecific(s3h_thread_key) : 0;
+	if (!num) {
+		num = ++s3h_threads;
+		if (s3h_thread_key_ok && pthread_setspecific(s3h_thread_key, (void *)(uintptr_t)num) != 0)
+			return num;
+	}
+	return num;
+}
 
 static size_t blk_hash(const void *p)
 {
@@ -157,24 +208,31 @@ static size_t scratch_round(size_t n)
 	return n ? (n + g - 1) / g * g : g;
 }
 
-/* hipFree every idle block of device dev (all streams when stream_only
- * is 0, else only those of `stream`), after the work using them is done.
- * Called with the lock held. */
-static void scratch_trim_locked(int dev, int stream_only, void *stream)
+/* Which idle blocks a trim frees: all, those of one stream (as this thread
+ * names it), or those of threads that have ended. */
+enum trim { TRIM_ALL, TRIM_STREAM, TRIM_GONE };
+
+/* hipFree those idle blocks of device dev, after the work using them is
+ * done. Called with the lock held. */
+static void scratch_trim_locked(int dev, enum trim what, void *stream)
 {
+	const unsigned owner = what == TRIM_STREAM ? stream_owner(stream) : 0;
 	int synced = 0;
 	for (int i = s3h_nblks - 1; i >= 0; i--) {
 		struct s3h_blk *b = &s3h_blks[i];
-		if (b->busy || b->dev != dev || (stream_only && b->stream != stream))
+		if (b->busy || b->dev != dev ||
+		    (what == TRIM_STREAM && (b->stream != stream || b->owner != owner)) ||
+		    (what == TRIM_GONE && b->owner != S3H_OWNER_GONE))
 			continue;
 		if (!synced) {
-			if (stream_only)
+			if (what == TRIM_STREAM)
 				(void)hipStreamSynchronize((hipStream_t)stream);
 			else
 				(void)hipDeviceSynchronize();
 			synced = 1;
 		}
 		(void)hipFree(b->p);
+		s3h_ngone -= b->owner == S3H_OWNER_GONE;
 		s3h_blks[i] = s3h_blks[--s3h_nblks];
 	}
 	/* slots moved: rebuild the idle list and the address index */
@@ -193,10 +251,11 @@ enum sam3_error s3h_scratch_alloc(void **p, size_t nbytes, void *stream)
 	const size_t most = need * 2 > need + ((size_t)4 << 20) ? need * 2 : need + ((size_t)4 << 20);
 	*p = NULL;
 	pthread_mutex_lock(&s3h_blk_lock);
+	const unsigned owner = stream_owner(stream);
 	int best = -1;
 	for (int j = 0; j < s3h_nidle; j++) {
 		const struct s3h_blk *b = &s3h_blks[s3h_idle[j]];
-		if (b->dev == dev && b->stream == stream && b->n >= need && b->n <= most &&
+		if (b->dev == dev && b->stream == stream && b->owner == owner && b->n >= need && b->n <= most &&
 		    (best < 0 || b->n < s3h_blks[s3h_idle[best]].n))
 			best = j;
 	}
@@ -208,6 +267,8 @@ enum sam3_error s3h_scratch_alloc(void **p, size_t nbytes, void *stream)
 		pthread_mutex_unlock(&s3h_blk_lock);
 		return SAM3_OK;
 	}
+	if (s3h_ngone)
+		scratch_trim_locked(dev, TRIM_GONE, NULL);
 	if (s3h_nblks == s3h_capblks) {
 		const int cap = s3h_capblks ? s3h_capblks * 2 : 64;
 		struct s3h_blk *t = realloc(s3h_blks, (size_t)cap * sizeof(*t));
@@ -235,14 +296,14 @@ enum sam3_error s3h_scratch_alloc(void **p, size_t nbytes, void *stream)
 	hipError_t e = hipMalloc(&q, need);
 	if (e == hipErrorOutOfMemory) {
 		(void)hipGetLastError();
-		scratch_trim_locked(dev, 0, NULL);
+		scratch_trim_locked(dev, TRIM_ALL, NULL);
 		e = hipMalloc(&q, need);
 	}
 	if (e != hipSuccess) {
 		pthread_mutex_unlock(&s3h_blk_lock);
 		return s3h_hip(e, "scratch");
 	}
-	s3h_blks[s3h_nblks++] = (struct s3h_blk){q, need, stream, dev, 1};
+	s3h_blks[s3h_nblks++] = (struct s3h_blk){q, need, stream, owner, dev, 1};
 	if (!s3h_bix_dirty && 2 * (size_t)s3h_nblks < s3h_bix_cap)
 		bix_put(s3h_nblks - 1);
 	else
@@ -262,6 +323,7 @@ enum sam3_error s3h_scratch_free(void *p, void *stream)
 		if (s3h_blks[i].busy) {
 			s3h_blks[i].busy = 0;
 			s3h_blks[i].stream = stream; /* its last use was enqueued here */
+			s3h_blks[i].owner = stream_owner(stream);
 			(void)idle_push(i); /* room was reserved when the block was made */
 		}
 		pthread_mutex_unlock(&s3h_blk_lock);
@@ -277,7 +339,7 @@ void s3h_scratch_release(void *stream)
 	int dev = 0;
 	(void)hipGetDevice(&dev);
 	pthread_mutex_lock(&s3h_blk_lock);
-	scratch_trim_locked(dev, 1, stream);
+	scratch_trim_locked(dev, TRIM_STREAM, stream);
 	pthread_mutex_unlock(&s3h_blk_lock);
 }
 

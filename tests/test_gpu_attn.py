@@ -16,6 +16,7 @@ checkers here:
     row returns zeros, Sk = 0 returns zeros.
 """
 import ctypes as C
+import threading
 from pathlib import Path
 
 import numpy as np
@@ -438,3 +439,74 @@ def test_sdpa_max_is_of_scores_that_count(env, dt, planes):
     mask[:, 32:] = -np.inf
     got, ref = run(dt, q, k, v, mask, path=MFMA)
     check(dt, got, ref, f"masked scores of +200, planes {planes}")
+
+
+PER_THREAD = C.c_void_p(2)  # hipStreamPerThread
+
+
+def in_thread(fn):
+    out = []
+    t = threading.Thread(target=lambda: out.append(fn()))
+    t.start()
+    t.join()
+    return out[0]
+
+
+def test_scratch_of_per_thread_streams():
+    """hipStreamPerThread is one handle for a stream per thread: a block one
+    thread gave back is not handed to another, whose stream does not wait
+    for its last use. A block of an ordinary stream is, and the giving
+    thread gets its own back; blocks of an ended thread do not get lost."""
+    lib = hip.load()
+    alloc, free = lib.s3h_scratch_alloc, lib.s3h_scratch_free
+    alloc.argtypes, free.argtypes = [C.POINTER(C.c_void_p), C.c_size_t, C.c_void_p], [C.c_void_p] * 2
+
+    def take(stream, n=3 << 20):
+        p = C.c_void_p()
+        hip.check(alloc(C.byref(p), n, stream), "scratch")
+        hip.check(free(p, stream), "scratch free")
+        return p.value
+
+    st = C.c_void_p()
+    hip.check(lib.sam3_hip_stream_create(C.byref(st)), "stream")
+    try:
+        mine = take(PER_THREAD)
+        assert in_thread(lambda: take(PER_THREAD)) != mine
+        assert take(PER_THREAD) == mine
+        shared = take(st)
+        assert in_thread(lambda: take(st)) == shared
+        for _ in range(3):  # each thread's block is freed by the next one's request
+            assert in_thread(lambda: take(PER_THREAD)) != mine
+        assert take(PER_THREAD) == mine
+    finally:
+        lib.s3h_scratch_release(PER_THREAD)
+        lib.sam3_hip_stream_destroy(st)
+
+
+def test_sdpa_planes_on_per_thread_streams(env):
+    """f32 attention with planes from two threads at once, each on its own
+    stream by the one handle: the results of separate calls."""
+    env.set("SAM3_HIP_ATTN_PLANES", "1")
+    lib, BH, Sq, Sk = hip.load(), 8, 300, 1000
+    sets, wants = [], []
+    for i in range(2):
+        q, k, v = inputs(1400 + 10 * i, BH, Sq, Sk, 64)
+        wants.append(hip.sdpa(q, k, v, None, dtype=abi.F32, path=MFMA))
+        sets.append([hip.DeviceBuffer.of(x) for x in (q, k, v)] + [hip.DeviceBuffer(q.nbytes)])
+    bad = []
+
+    def work(i):
+        q, k, v, o = sets[i]
+        for _ in range(30):
+            hip.check(lib.sam3_hip_sdpa(abi.F32, q.ptr, k.ptr, v.ptr, None, o.ptr, BH, Sq, Sk, 64,
+                                        PER_THREAD), "sdpa")
+            hip.check(lib.sam3_hip_stream_synchronize(PER_THREAD), "sync")
+            if not np.array_equal(o.download(np.float32, wants[i].shape), wants[i]):
+                bad.append(i)
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not bad
