@@ -288,7 +288,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dlq8(GemmArgs p)
 	if (again)
 		q8_wauto_scale<FM, FN>(acc, fe, smem, lane, wn0);
 	__syncthreads();
-	write_tile_ck<FM, FN, WTN, S3K_F32, true>(p, acc, smem, wave, lane, tm * BM + wm0, tn * BN + wn0, bz);
+	write_tile_ck<FM, FN, WTN, S3K_F32, true, false, false>(p, acc, smem, wave, lane, tm * BM + wm0, tn * BN + wn0, bz);
 }
 
 /*
@@ -525,7 +525,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 1) gemm_dlpq(GemmArgs p)
 	if (again)
 		q8_wauto_scale<FM, FN>(acc, fe, smem, lane, wn0);
 	__syncthreads();
-	write_tile_ck<FM, FN, WTN, S3K_F32, true>(p, acc, smem, wave, lane, tm * BM + wm0,
+	write_tile_ck<FM, FN, WTN, S3K_F32, true, false, false>(p, acc, smem, wave, lane, tm * BM + wm0,
 						 tn * BN + wn0, bz);
 }
 
