@@ -107,6 +107,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) conv_dl(ConvArgs q)
 	/* Tap walk of the next k-step to issue (steps are issued in order):
 	 * plane seg, tap (kh, kw), first channel ic. */
 	int w_seg = 0, w_kh = 0, w_kw = 0, w_ic = 0;
+	const KOff<split_f32<FAM, CK>()> ko(p);
 	auto issue = [&](int kt) {
 		const int k0 = kt * BK;
 		const unsigned st = lds0 + (unsigned)((kt % STAGES) * SB) + (unsigned)wave * 1024u;
@@ -120,7 +121,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) conv_dl(ConvArgs q)
 		}
 #pragma unroll
 		for (int j = 0; j < B_PER; ++j)
-			dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b<split_f32<FAM, CK>()>(p, k0));
+			dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], ko.b(k0));
 		w_ic += BK;
 		if (w_ic == q.C) {
 			w_ic = 0;

@@ -112,20 +112,26 @@ constexpr bool split_f32()
 	return FAM == FAM_BF16 && (CK == S3K_F32 || CK == S3K_C_PLANES);
 }
 
-/* Byte offset of k in a row of A or W: 2k, or (SEG) its place in the two
- * planes that k walks as hi, lo, hi (A) and hi, hi, lo (W). Steps never
- * straddle a plane (kseg is a multiple of 64). */
+/* Byte offset of k in a row of A (a) or W (b): 2k, or (SEG) its place in
+ * the two planes that k walks as hi, lo, hi (A) and hi, hi, lo (W): past
+ * 2 * kseg, or kseg, it starts over. Steps never straddle a plane (kseg is
+ * a multiple of 64). */
 template <bool SEG>
-__device__ __forceinline__ unsigned k_off_a(const GemmArgs &p, int k)
-{
-	return 2u * (unsigned)(SEG && p.kseg && k >= 2 * p.kseg ? k - 2 * p.kseg : k);
-}
-
-template <bool SEG>
-__device__ __forceinline__ unsigned k_off_b(const GemmArgs &p, int k)
-{
-	return 2u * (unsigned)(SEG && p.kseg && k >= p.kseg ? k - p.kseg : k);
-}
+struct KOff {
+	int ta, tb;
+	__device__ __forceinline__ explicit KOff(const GemmArgs &p)
+		: ta(SEG && p.kseg ? 2 * p.kseg : 0x7FFFFFFF), tb(SEG && p.kseg ? p.kseg : 0x7FFFFFFF)
+	{
+	}
+	__device__ __forceinline__ unsigned a(int k) const
+	{
+		return 2u * (unsigned)(SEG && k >= ta ? k - ta : k);
+	}
+	__device__ __forceinline__ unsigned b(int k) const
+	{
+		return 2u * (unsigned)(SEG && k >= tb ? k - tb : k);
+	}
+};
 
 /* Workgroup id -> (tile_m, tile_n). Workgroups are dealt round-robin to
  * the 8 XCDs; ids are regrouped so each XCD gets a contiguous range of

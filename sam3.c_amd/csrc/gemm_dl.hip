@@ -96,16 +96,17 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dl(GemmArgs p)
 	/* A whole k-step moves every lane's chunk by 2*k0 bytes: that goes in
 	 * the scalar offset (rows past M/N keep an offset past the range). Only
 	 * a k-step that crosses K selects chunks per lane. */
+	const KOff<split_f32<FAM, CK>()> ko(p);
 	auto issue = [&](int kt) {
 		const int k0 = kt * BK;
 		const unsigned st = lds0 + (unsigned)((kt % STAGES) * SB) + (unsigned)wave * 1024u;
 		if (k0 + BK <= p.K) {
 #pragma unroll
 			for (int j = 0; j < A_PER; ++j)
-				dma16s(st + j * NW * 1024, ra, a_off[j], k_off_a<split_f32<FAM, CK>()>(p, k0));
+				dma16s(st + j * NW * 1024, ra, a_off[j], ko.a(k0));
 #pragma unroll
 			for (int j = 0; j < B_PER; ++j)
-				dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], k_off_b<split_f32<FAM, CK>()>(p, k0));
+				dma16s(st + A_BYTES + j * NW * 1024, rb, b_off[j], ko.b(k0));
 		} else {
 #pragma unroll
 			for (int j = 0; j < A_PER; ++j) {
@@ -243,13 +244,14 @@ __global__ void __launch_bounds__(64 * WGM * WGN, 1) gemm_dlp(GemmArgs p)
 		off[t] = g < (isa ? p.M : p.N) ? (unsigned)(g * (isa ? p.lda_b : p.ldb_b) + c * 16)
 					       : S3K_OOB;
 	}
+	const KOff<split_f32<FAM, CK>()> ko(p);
 	auto dma = [&](int kt, int t, int stg) {
 		if (t < A_PER)
 			dma16s(lds0 + (unsigned)(stg * A_BYTES + (t * NW + wave) * 1024), ra, off[t],
-			       k_off_a<split_f32<FAM, CK>()>(p, kt * BK));
+			       ko.a(kt * BK));
 		else
 			dma16s(lds0 + (unsigned)(B_BASE + stg * B_BYTES + ((t - A_PER) * NW + wave) * 1024),
-			       rb, off[t], k_off_b<split_f32<FAM, CK>()>(p, kt * BK));
+			       rb, off[t], ko.b(kt * BK));
 	};
 
 	unsigned abase[4], bbase[4];
