@@ -46,7 +46,8 @@ __device__ __forceinline__ int cv_off(int row, int c)
 }
 
 template <int BM, int BN, int BK, int WGM, int WGN, int STAGES, int FAM, int CK, int OCC>
-__global__ void __launch_bounds__(64 * WGM * WGN, OCC) conv_dl(ConvArgs q)
+__global__ void __launch_bounds__(64 * WGM * WGN, OCC > 1 ? OCC : (dl_waves<WGM * WGN, STAGES * (BM + BN) * BK * 2, CK>()))
+conv_dl(ConvArgs q)
 {
 	const GemmArgs &p = q.g;
 	constexpr int NW = WGM * WGN;

@@ -112,6 +112,17 @@ constexpr bool split_f32()
 	return FAM == FAM_BF16 && (CK == S3K_F32 || CK == S3K_C_PLANES);
 }
 
+/* Waves per SIMD to leave registers for: those of as many workgroups of NW
+ * waves as the LDS has room for. Two of 192x128 (8 waves, 80 KiB) need 128
+ * registers or fewer; without the bound the 16-bit and planes outputs took
+ * 129-130 and a CU held one. (The f16 operand takes 135: bounded it spills
+ * five.) */
+template <int NW, int LDS, int CK>
+constexpr int dl_waves()
+{
+	return CK == S3K_C_F16OP ? NW / 4 : 160 * 1024 / LDS * NW / 4;
+}
+
 /* Byte offset of k in a row of A (a) or W (b): 2k, or (SEG) its place in
  * the two planes that k walks as hi, lo, hi (A) and hi, hi, lo (W): past
  * 2 * kseg, or kseg, it starts over. Steps never straddle a plane (kseg is

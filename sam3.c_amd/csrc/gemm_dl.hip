@@ -46,7 +46,8 @@ __host__ __device__ constexpr bool qkv_tiles(int ck, int wtn)
 }
 
 template <int BM, int BN, int BK, int WGM, int WGN, int STAGES, int FAM, int CK, int OCC>
-__global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dl(GemmArgs p)
+__global__ void __launch_bounds__(64 * WGM * WGN, OCC > 1 ? OCC : (dl_waves<WGM * WGN, STAGES * (BM + BN) * BK * 2, CK>()))
+gemm_dl(GemmArgs p)
 {
 	constexpr int NW = WGM * WGN;
 	constexpr int CPR = BK / 8;
@@ -208,7 +209,7 @@ __global__ void __launch_bounds__(64 * WGM * WGN, OCC) gemm_dl(GemmArgs p)
 
 /* QKV: the S3K_EPI_QKV epilogue (f32 output), instead of C */
 template <int BM, int BN, int WGM, int WGN, int FAM, int CK, bool INTER, bool QKV = false>
-__global__ void __launch_bounds__(64 * WGM * WGN, 1) gemm_dlp(GemmArgs p)
+__global__ void __launch_bounds__(64 * WGM * WGN, (dl_waves<WGM * WGN, 2 * (BM + BN) * 128, CK>())) gemm_dlp(GemmArgs p)
 {
 	constexpr int NW = WGM * WGN, BK = 64, CPR = 8;
 	constexpr int A_BYTES = BM * BK * 2, B_BYTES = BN * BK * 2; /* one stage */
