@@ -410,13 +410,19 @@ extern "C" int s3k_conv_implicit(const struct s3k_conv *c, const void *xa, const
 	 * not cover the 256 CUs (72x72 maps: 5184 x 256), else the GEMM's
 	 * rule (256x256 for one nearly full round, 192x128 from 192 tiles).
 	 * The 64x64 tiles keep three k-steps in flight (four stages, two
-	 * workgroups per CU up to 512 tiles, three stages above): 1x1 over
-	 * 72x72x1024 (k' 3072) 26.6 -> 22.6 us, 3x3 over 72x72x256 47.8 ->
-	 * 45, over 36x36x256 (84 tiles, 108 k-steps) 45 -> 28. */
+	 * workgroups per CU up to 512 tiles, three stages above): f32 1x1
+	 * over 72x72x1024 (k' 3072) 26.6 -> 22.6 us, 3x3 over 72x72x256 47.8
+	 * -> 45, over 36x36x256 (84 tiles, 108 k-steps) 45 -> 28; bf16 3x3
+	 * over 36x36x256 with operands out of HBM 27.0 -> 14.6, out of the
+	 * MALL 19.8 -> 14.4. Where one call after another finds both operands
+	 * in L2 the two-stage ring is ahead (the same, 13.4 against 14.7): a
+	 * model's convolutions run once per image and do not. Up to three
+	 * steps there is nothing to keep in flight: 64 channels 1x1 over
+	 * 48x48, f32 8.8-9.9 on two stages, 9.4-10.0 on four. */
 	if (cfg < 0) {
 		const long long t9 = conv_tiles(q.g.M, q.g.N, 256, 256), t10 = conv_tiles(q.g.M, q.g.N, 192, 128);
 		const long long t6 = conv_tiles(q.g.M, q.g.N, 64, 64);
-		cfg = conv_tiles(q.g.M, q.g.N, 128, 128) < 256 ? (t6 <= 512 ? 6 : 7) : (t9 >= 224 && t9 <= 256) ? 9 : t10 >= 192 ? 10 : 4;
+		cfg = conv_tiles(q.g.M, q.g.N, 128, 128) < 256 ? (q.g.K <= 3 * 64 ? 2 : t6 <= 512 ? 6 : 7) : (t9 >= 224 && t9 <= 256) ? 9 : t10 >= 192 ? 10 : 4;
 	}
 	switch (cfg) {
 	case 2:  return launch_conv_cfg<64, 64, 64, 2, 2, 2, 2>(q, c->kind, st);
