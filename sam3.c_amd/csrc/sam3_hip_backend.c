@@ -963,6 +963,7 @@ static enum sam3_error run_matmul(struct sam3_hip_backend *hb, const struct sam3
 				for (int t = 0; t < qcs[y].n; t++)
 					done[qcs[y].idx[t]] = 1;
 				n_chain += qcs[y].n;
+				hb->stats.operand_writes += (qkv.planes >> y) & 1;
 			}
 	} else if (o_fmt != S3H_A_PLAIN) {
 		/* an f16 operand carries its row tags (two words per row) after

@@ -1005,13 +1005,16 @@ def test_vit_block_full_size_global(env, wkind):
 def test_qkv_gemm_stores_key_and_value_planes(env, wkind, grid, window, is_global):
     """A ViT block whose qkv GEMM stores K and V as the bf16 planes its
     attention reads, where the kernel choice allows (36 and 196 keys; 81
-    keys keep the few-keys kernel): the same bits as f32 K and V
-    (SAM3_HIP_ATTN_PLANES=0)."""
+    keys keep the few-keys kernel): two operand writes more than with
+    SAM3_HIP_ATTN_PLANES=0, and the same bits as f32 K and V."""
     def run(mode):
         env.set("SAM3_HIP_ATTN_PLANES", mode)
-        return small_vit_block(wkind, grid, window, is_global)
+        writes = []
+        return small_vit_block(wkind, grid, window, is_global, writes=writes), writes
 
-    a, b = run("-1"), run("0")
+    (a, wa), (b, wb) = run("-1"), run("0")
+    keys = (grid if is_global else window) ** 2
+    assert [x - y for x, y in zip(wa, wb)] == [0 if 64 < keys <= 128 else 2] * 2
     assert np.isfinite(a).all() and np.array_equal(a.view(np.uint32), b.view(np.uint32))
 
 
@@ -1054,8 +1057,9 @@ def small_vit_graph(wkind, grid, window, is_global, e=256, heads=4):
     return G, graph.vit_block(G, x, p, heads, grid, window, is_global, tc, ts)
 
 
-def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
-    """Output of one ViT block of width e, evaluated twice on one backend."""
+def small_vit_block(wkind, grid, window, is_global, e=256, heads=4, writes=None):
+    """Output of one ViT block of width e, evaluated twice on one backend;
+    appends each eval's count of operand writes to `writes`."""
     npos = grid * grid
     G, out = small_vit_graph(wkind, grid, window, is_global, e, heads)
     be = hip.Backend(0)
@@ -1064,6 +1068,8 @@ def small_vit_block(wkind, grid, window, is_global, e=256, heads=4):
         for _ in range(2):  # the second eval reuses the allocations
             assert be.graph_eval(G.g) == abi.OK
             assert be.stats().host_nodes == 0
+            if writes is not None:
+                writes.append(be.stats().operand_writes)
             res.append(np.ctypeslib.as_array(C.cast(out.data, C.POINTER(C.c_float)),
                                              shape=(npos, e)).copy())
     finally:
