@@ -371,6 +371,15 @@ def test_sdpa_graph_eval_2d():
 
 
 # ------------------------------------- f32 over prepared K and V planes
+def planes_want(BH, Sq, Sk, masked):
+    """Bytes of planes an f32 call on the MFMA kernel makes first (0: none)."""
+    want = hip.load().s3k_attn_planes_want
+    want.restype = C.c_size_t
+    want.argtypes = [C.c_int] * 2 + [C.c_void_p] * 5 + [C.c_int] * 6
+    p = 1 << 20
+    return want(MFMA, abi.F32, p, p, p, p if masked else None, p, BH, Sq, Sk, 64, 0, 0)
+
+
 @pytest.mark.parametrize("masked", [False, True], ids=["nomask", "mask"])
 @pytest.mark.parametrize("BH,Sq,Sk", [(1, 1, 1), (3, 150, 65), (9, 129, 64), (2, 257, 448),
                                       (2, 31, 449), (3, 130, 640), (1, 200, 1001)])
@@ -389,9 +398,11 @@ def test_sdpa_planes(env, BH, Sq, Sk, masked):
         mask[Sq // 2, :] = -np.inf
         mask[Sq // 3, : Sk // 2] = -3.4028234e38
     env.set("SAM3_HIP_ATTN_PLANES", "1")
+    assert planes_want(BH, Sq, Sk, masked) == BH * Sk * 512  # the scratch a call fills first
     got, ref = run(abi.F32, q, k, v, mask, path=MFMA)
     check(abi.F32, got, ref, f"planes {BH}x{Sq}x{Sk} {masked}")
     env.set("SAM3_HIP_ATTN_PLANES", "0")
+    assert planes_want(BH, Sq, Sk, masked) == 0
     plain, _ = run(abi.F32, q, k, v, mask, path=MFMA)
     if Sk <= 448:
         assert np.array_equal(got.view(np.uint32), plain.view(np.uint32))

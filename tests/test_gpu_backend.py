@@ -219,13 +219,14 @@ def _view(big, nbytes, dtype):
 def test_reused_host_address_copies_only_the_tensor_bytes(be):
     """sam3.c recycles arena memory between graphs without cache_invalidate
     (image_encoder.c:737-738). Eval 1 leaves at host address B a residency
-    entry for fc1's output, written as fc2's bf16-planes operand (6 bytes per
-    element on the device for a 4-byte-per-element host tensor). Eval 2's final
+    entry for fc1's output, written as fc2's bf16-planes operand: rows of 520
+    values, no whole number of 64-k steps, so three planes, 6 bytes per
+    element on the device for a 4-byte-per-element host tensor. Eval 2's final
     output is a smaller f32 tensor at the same B: its readback must write
     exactly its own bytes, and the next eval's ephemeral input at B must be
     uploaded with exactly its own bytes."""
     O = oracle()
-    M, K, N1, N2, N3 = 256, 256, 512, 256, 128
+    M, K, N1, N2, N3 = 256, 256, 520, 256, 128
     big = np.full(M * N1 * 6 + 4096, 0x7F, np.uint8)
     x = synth.randn(11, (M, K))
     w1 = synth.randn(12, (N1, K), 0.05)
