@@ -77,8 +77,9 @@ struct sam3_hip_eval_stats {
 	int mapped_reads;  /* inputs read from a range mapped by map_weights   */
 	int prep_hits;     /* weights whose prepared copy (bf16 planes, padded
 			    * rows) was reused instead of recomputed           */
-	int operand_writes; /* LAYERNORM outputs written straight in the form
-			     * their one consuming GEMM reads (not kept)      */
+	int operand_writes; /* outputs written straight in the form their one
+			     * reader takes (not kept): a GEMM's A, a
+			     * convolution's planes, attention's K and V      */
 	int range_reruns;  /* 1 when a fused producer's f16 GEMM operand held
 			    * values outside the f16 range and the graph was
 			    * run again with f32 operands (then the counts
@@ -380,7 +381,15 @@ enum sam3_error sam3_hip_matmul_on_path(int path, int a_dtype, const void *a,
  * aligned tensors runs the MFMA kernel (f32 as three bf16 products per
  * step: hi*hi + lo*hi + hi*lo), or for f32 with at most 128 keys a
  * latency-bound kernel in plain f32 arithmetic (the text encoder's
- * attention); other D up to 512 run a one-wave-per-row f32 kernel. */
+ * attention); other D up to 512 run a one-wave-per-row f32 kernel.
+ * In f32 a call may first split K and V into bf16 planes, once instead of
+ * once per 128 queries, where that was measured to pay (long sequences,
+ * masks): this takes 512 bytes per key and head of the library's device
+ * scratch for `stream`, allocated when a size is first seen. A call that
+ * cannot have it, or whose stream is being captured into a graph, splits
+ * them as it reads them: the same bits where the keys are not shared out
+ * among wave groups, f32 rounding apart elsewhere, and slower (16 heads,
+ * 1369 queries and keys, with a mask: 121 against 51 us). */
 enum sam3_error sam3_hip_sdpa(int dtype, const void *q, const void *k, const void *v,
 			      const float *mask, void *out, int BH, int Sq, int Sk, int D,
 			      void *stream);

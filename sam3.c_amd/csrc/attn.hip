@@ -1000,8 +1000,9 @@ __global__ void __launch_bounds__(256 * KS, KS > 1 ? 1 : MASK ? 2 : 3) attn_plan
 
 	if constexpr (KS > 1) {
 		/* merge: the groups g > 0 leave their 34 floats per lane in LDS
-		 * ([value][lane], one 8.5 KiB region per wave, in the K slots no
-		 * wave reads any more), group 0 adds them in order */
+		 * ([value][lane], one 8.5 KiB region per wave, from offset 0 over
+		 * the groups' K and V slots, which no wave reads past this
+		 * barrier), group 0 adds them in order */
 		__syncthreads();
 		constexpr int REG = 34 * 64 * 4;
 		static_assert((KS - 1) * 4 * REG <= KS * AP_GROUP, "merge regions fit");

@@ -947,11 +947,15 @@ extern "C" int s3k_dl_eligible(const struct s3k_gemm *g)
  *     13.6 here; 576x1024x4096 31.8 -> 20.2 (144 tiles), 169x768x3072
  *     24.9 -> 15.5 (36), 5184x512x512 8.1 -> 7.0 (648). Past 768 tiles
  *     the larger tiles' fewer L2 bytes win (2500x2048x512, 1280 tiles:
- *     10.7 here, 9.6 on 192x128). With K % 64 != 0 the line lies at 512:
- *     rows then start off the 128-byte lines and the small tiles' larger
- *     L2 traffic costs more (700x4096x1544, 704 tiles: 22.4 us here, 18.5
- *     on 128x128; 2304x1024x2056 28.1 and 28.8; with K % 64 == 0
- *     700x4096x2048 21.4 and 23.4);
+ *     10.7 here, 9.6 on 192x128). From 513 to 768 it is ahead of the
+ *     128x128 tiles of cfg 4 at every K (2560x1024x1024 11.5 and 12.9 us,
+ *     x4096 38.4 and 41.8); their pipelined form (cfg 26) is ahead of it
+ *     up to K 1024 (10.4) and behind from K 2048 (22.3 and 20.8). With
+ *     K % 64 != 0 the line lies at 512: rows then start off the 128-byte
+ *     lines, and past it the better tile depends on the shape, 128x128
+ *     for few long rows (700x4096x1544: 18.5 against 22.4 us here), this
+ *     by less for many (2560x1024x1544: 23.7 and 22.1; 3072x1024x1544
+ *     24.0 and 23.4);
  *   - 128x128 (cfg 4, 4 waves) between that and 192 tiles of 192x128.
  *   - K = 64 with M, N multiples of 192 and at least 1024 such tiles
  *     (attention scores over many slices): the persistent gemm_dlk,

@@ -982,9 +982,8 @@ __global__ void __launch_bounds__(1024) q8_gemv(StreamArgs p)
 }
 
 /*
- * q8_gemv_rows4: q8_gemv<1, 16> on four weight rows per workgroup, for a
- * launch whose 16-row groups would leave CUs idle (fc2 and proj of the
- * text encoder at one token: 64 groups on 256 CUs). Such a launch lasts as
+ * q8_gemv_rows4: q8_gemv<1, 16> on four weight rows per workgroup, for up
+ * to 4096 rows (256 of q8_gemv's 16-row groups). Such a launch lasts as
  * long as one workgroup: start, first bytes, then a barrier and the ring's
  * steps per chunk of 16 k-blocks. Here a quarter of the bytes fall to a
  * workgroup and they all fit the LDS, so every load is issued at the
@@ -992,8 +991,12 @@ __global__ void __launch_bounds__(1024) q8_gemv(StreamArgs p)
  * either. q8_gemv's 16 waves become 16 groups of 16 lanes (four rows x
  * four k-octets), each walking the same blocks in the same order, and the
  * sums are added in the same order: the same bits. K % 512 == 0, K <=
- * 4096, N % 4 == 0; bias, GELU and residual. Four encoder layers of one
- * token, whose fc2 (N 1024, K 4096) it runs: 98.7 -> 89.3 us.
+ * 4096, N % 4 == 0; bias, GELU and residual. What it gains grows with K:
+ * one row x 4096, N 64-4096, 5.3-5.6 -> 4.0-4.2 us a launch (fc2 of the
+ * text encoder at one token: N 1024); up to K 2048 both take the 4.1 us
+ * of a launch. Past 4096 rows q8_gemv's groups fill the CUs: 4100 x 4096
+ * 9.3 us there. qkv, proj and fc1 of that encoder form their input row
+ * from a LayerNorm or the attention and stay on q8_gemv.
  */
 constexpr int G4_KMAX = 4096;
 
