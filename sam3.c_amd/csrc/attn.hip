@@ -706,12 +706,13 @@ __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_f
  *     per-lane loads would touch 32 rows, i.e. 32 cache lines, with each
  *     instruction.
  * Bound by the MFMAs and the softmax's VALU work on the busiest CUs: 16 x
- * 5184 x 5184 318 us against 400 for attn_fwd (1038 TFLOP/s of bf16 MFMA;
- * counters: MFMA busy 52 %, VALU 40 % of the time, 656 workgroups on 768
- * places), 144 heads x 576 44.7 against 55.2, masked 16 x 1369 47 against
- * 120. Registers matter: the order of finish_half(1) and settle(0) below
- * decides whether the kernel spills at 168 (then 155 us where it takes
- * 105). */
+ * 5184 x 5184 319 us, attn_planes_k included, against 382 for attn_fwd
+ * (1036 TFLOP/s of bf16 MFMA; counters: MFMA busy 51 %, VALU 40 % of the
+ * time, 656 workgroups on 768 places), masked 16 x 1369 51 against 108;
+ * 144 heads x 576 over planes that are already stored 44.7 against 55.2
+ * (another run, attn_planes_k included: 55.0 against 48.6). Registers
+ * matter: the order of finish_half(1) and settle(0) below decides whether
+ * the kernel spills at 168 (then 155 us where it takes 105). */
 constexpr int AP_TILE = 2 * AT_K_BYTES;              /* hi and lo, 16 KiB */
 constexpr int AP_GROUP = 3 * AP_TILE;                /* K, K, V */
 constexpr int AP_MASK = 32 * AT_BKV * 4;             /* one wave's mask tile */
