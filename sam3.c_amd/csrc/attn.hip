@@ -182,6 +182,26 @@ struct at_int {
  * then below 2^15, inside the f16 range. */
 constexpr float AT_PSUM_MAX = 32768.0f;
 
+/* The max m is moved to when half 0 of a tile is redone also covers half 1,
+ * whose scores are then still without their mask and with zeros for keys
+ * past Sk: m may pass the scores that count, by up to 2^AT_SLACK. All
+ * probabilities then carry a factor down to 2^-AT_SLACK, which the division
+ * by their sum takes out: exact in the exponent range of f32 and bf16; in
+ * f16 it costs 8 of the 24 binary places between 1 and the smallest
+ * subnormal. Past the slack (scores of -200 beside a key that does not
+ * exist) it would turn them all into zeros: half 0 then takes its own max. */
+template <int DT>
+constexpr float AT_SLACK = DT == S3K_F16 ? 8.0f : 64.0f;
+
+template <int DT>
+__device__ __forceinline__ float at_new_max(float m_run, float own, float other, bool other_counts)
+{
+	constexpr float LOG2E = 1.44269504088896341f;
+	const float mo = fmaxf(m_run, at_max_pair(own) * LOG2E);
+	const float ma = fmaxf(mo, at_max_pair(other) * LOG2E);
+	return !other_counts && ma - mo > AT_SLACK<DT> ? mo : ma;
+}
+
 /* Normalize (a query with no finite score keeps zeros, as the reference's
  * row_sum > 0 test leaves it) and store out[q][d] from a wave's O^T. */
 template <int DT>
@@ -585,27 +605,26 @@ __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_f
 				return ts;
 			};
 			/* if some lane's sum passed the bound: move the max to the
-			 * tile's, rescale what is accumulated, redo half mb (rare).
-			 * The scores of half 1 are still raw in settle(0): with a mask,
-			 * or keys past Sk in the tile, each half takes its own max, as
-			 * the raw score of a key that does not count could raise the
-			 * max until every real probability is 0. (Finishing half 1
-			 * before settle(0) takes 162 registers instead of 120; in a
-			 * copy inside it, 400 heads of 49 bf16 tokens take 5.9 us
-			 * instead of 5.4.) */
+			 * tile's (at_new_max), rescale what is accumulated, redo half
+			 * mb (rare). In settle(0) half 1's scores count as they are
+			 * before its mask and range. Without a mask half 1 is finished
+			 * after settle(0) (before it the kernel takes 162 registers
+			 * instead of 120); with one before it, the raw maximum kept in
+			 * raw1 (180 registers instead of 212: 16 x 1369 x 1369 bf16
+			 * 79.2 us instead of 83.0). */
 			const bool whole = !MASK && kbase + AT_BKV <= p.Sk;
+			auto half_max = [&](int mb) {
+				float mt = s[mb][0];
+#pragma unroll
+				for (int r = 1; r < 16; ++r)
+					mt = fmaxf(mt, s[mb][r]);
+				return mt;
+			};
+			float raw1 = 0.0f;
 			auto settle = [&](int mb, float ts) {
 				if (__builtin_amdgcn_ballot_w64(!(ts <= AT_PSUM_MAX))) {
-					float mt = s[mb][0];
-#pragma unroll
-					for (int r = 1; r < 16; ++r)
-						mt = fmaxf(mt, s[mb][r]);
-					if (whole) {
-#pragma unroll
-						for (int r = 0; r < 16; ++r)
-							mt = fmaxf(mt, s[1 - mb][r]);
-					}
-					const float m_new = fmaxf(m_run, at_max_pair(mt) * LOG2E);
+					const float m_new = at_new_max<DT>(m_run, half_max(mb), MASK && !mb ? raw1 : half_max(1 - mb),
+									   mb || whole);
 					const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 					m_run = m_new;
 					l_run *= alpha;
@@ -650,8 +669,15 @@ __global__ void __launch_bounds__(64 * NW, (at_minb<DT, NW, MASK, VD>())) attn_f
 			finish_half(0);
 			scores_half(1);
 			const float ts0 = probs(0);
-			settle(0, ts0);
-			finish_half(1);
+			if constexpr (MASK) {
+				if (__builtin_amdgcn_ballot_w64(!(ts0 <= AT_PSUM_MAX)))
+					raw1 = half_max(1);
+				finish_half(1);
+				settle(0, ts0);
+			} else {
+				settle(0, ts0);
+				finish_half(1);
+			}
 			pv_half(0);
 			const float ts1 = probs(1);
 			settle(1, ts1);
@@ -911,22 +937,24 @@ __global__ void __launch_bounds__(256 * KS, KS > 1 ? 1 : MASK ? 2 : 3) attn_plan
 			}
 			return ts;
 		};
-		/* as attn_fwd: when some lane's sum passed the bound, move the max
-		 * to the tile's (to the half's where attn_fwd does so, for the same
-		 * bits), rescale, redo half mb */
+		/* as attn_fwd. One group takes attn_fwd's maxima, for its bits:
+		 * half 1's in settle(0) from before its mask and range were
+		 * applied. More groups, whose sums are merged in another order
+		 * anyway, take the finished scores'. */
 		const bool whole = !MASK && kbase + AT_BKV <= p.Sk;
+		auto half_max = [&](int mb) {
+			float mt = s[mb][0];
+#pragma unroll
+			for (int r = 1; r < 16; ++r)
+				mt = fmaxf(mt, s[mb][r]);
+			return mt;
+		};
+		float raw1 = 0.0f;
 		auto settle = [&](int mb, float ts) {
 			if (__builtin_amdgcn_ballot_w64(!(ts <= AT_PSUM_MAX))) {
-				float mt = s[mb][0];
-#pragma unroll
-				for (int r = 1; r < 16; ++r)
-					mt = fmaxf(mt, s[mb][r]);
-				if (whole) {
-#pragma unroll
-					for (int r = 0; r < 16; ++r)
-						mt = fmaxf(mt, s[1 - mb][r]);
-				}
-				const float m_new = fmaxf(m_run, at_max_pair(mt) * LOG2E);
+				const float m_new = at_new_max<S3K_F32>(m_run, half_max(mb),
+									KS > 1 || mb ? half_max(1 - mb) : raw1,
+									KS > 1 || mb || whole);
 				const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
 				m_run = m_new;
 				l_run *= alpha;
@@ -961,6 +989,8 @@ __global__ void __launch_bounds__(256 * KS, KS > 1 ? 1 : MASK ? 2 : 3) attn_plan
 			scores_half(1);
 			/* (finish before settle: the other order spills registers) */
 			ts0 = probs(0);
+			if (KS == 1 && __builtin_amdgcn_ballot_w64(!(ts0 <= AT_PSUM_MAX)))
+				raw1 = half_max(1);
 			finish_half(1);
 			settle(0, ts0);
 		}

@@ -452,6 +452,52 @@ def test_sdpa_max_is_of_scores_that_count(env, dt, planes):
     check(dt, got, ref, f"masked scores of +200, planes {planes}")
 
 
+@pytest.mark.parametrize("dt", DTS, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("planes", ["0", "1"])
+def test_sdpa_max_slack(env, dt, planes):
+    """Masked scores a little above the real ones, on both sides of the
+    slack (2^8 in f16, 2^64 else) that the running max may have over
+    scores that count: the usual bounds hold. Entries are exact in bf16, so
+    the scores are exact too."""
+    if dt != abi.F32 and planes == "1":
+        pytest.skip("planes are for f32")
+    env.set("SAM3_HIP_ATTN_PLANES", planes)
+    rng = np.random.default_rng(1297)
+    q = np.ones((1, 40, 64), np.float32)
+    v = synth.randn(1298, (1, 64, 64))
+    mask = np.zeros((40, 64), np.float32)
+    mask[:, 32:] = -np.inf
+    for above in (3.0, 5.0, 5.5, 7.0, 40.0, 44.0, 44.5, 48.0):
+        k = rng.integers(-2, 3, (1, 64, 64)).astype(np.float32) / 32
+        k[:, 32:] = above / 8
+        got, ref = run(dt, q, k, v, mask, path=MFMA)
+        check(dt, got, ref, f"masked scores of {above}, planes {planes}")
+
+
+@pytest.mark.parametrize("dt", DTS, ids=["f32", "bf16", "f16"])
+@pytest.mark.parametrize("planes", ["0", "1"])
+def test_sdpa_zero_mask_changes_no_bit(env, dt, planes):
+    """The same maxima whether or not a tile has a mask or an end: a mask of
+    zeros gives the bits of no mask, and keys past Sk those of zero keys
+    masked with -inf (tiles of 64 keys; the second has 23 or 32 + 23)."""
+    if dt != abi.F32 and planes == "1":
+        pytest.skip("planes are for f32")
+    env.set("SAM3_HIP_ATTN_PLANES", planes)
+    for Sk in (87, 119, 128):
+        q, k, v = inputs(1300 + Sk, 2, 70, 128, 64)
+        q *= 2.0
+        k[:, Sk:] = 0.0
+        mask = np.zeros((70, 128), np.float32)
+        full, _ = run(dt, q, k, v, path=MFMA)
+        zero, _ = run(dt, q, k, v, mask, path=MFMA)
+        assert np.array_equal(full.view(np.uint8), zero.view(np.uint8))
+        mask[:, Sk:] = -np.inf
+        masked, ref = run(dt, q, k, v, mask, path=MFMA)
+        ended, _ = run(dt, q, k[:, :Sk], v[:, :Sk], path=MFMA)
+        assert np.array_equal(masked.view(np.uint8), ended.view(np.uint8))
+        check(dt, masked, ref, f"{Sk} of 128 keys, planes {planes}")
+
+
 PER_THREAD = C.c_void_p(2)  # hipStreamPerThread
 
 
